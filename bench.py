@@ -371,8 +371,8 @@ def instationary_leg(pkg, n, k):
     return out
 
 
-# the 64^3 Q3 FP64 apply y = J z (constant kappa: the z-walk instance, template argument 2)
-APPLY_KERNEL = "dg_apply_rowreg_kernel<4, double, false, false, false, false, false, false, 2>"
+# the 64^3 Q3 FP64 apply y = J z (constant kappa): Q3, constant symmetric operator, y = J z
+APPLY_KERNEL = "dg_mfma_kernel<4, 0, 0>"
 CALIB_KERNEL = "axpy_kernel<double>"
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "apply_traffic.json")
 
@@ -430,7 +430,7 @@ def profile_summary(d, n, k):
 
 FP64_PEAK = 78.6e12  # MI355X dense FP64 (vector and matrix), FLOP/s
 APPLY_WORKLOADS = {  # grid size (threads) of the apply launches of this benchmark -> workload
-    "2097152": "64^3 Q3", "4194304": "64^3 Q3", "995328": "96^3 Q2", "7962624": "96^3 Q2",
+    "131072": "64^3 Q3", "442368": "96^3 Q2", "2097152": "64^3 Q3", "4194304": "64^3 Q3", "995328": "96^3 Q2", "7962624": "96^3 Q2",
     "56623104": "96^3 Q2"}  # the last: conv_var_kernel, one 64-lane wave per cell
 
 
@@ -461,7 +461,7 @@ def counter_summary(d):
         dur[r["Kernel_Name"]].append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
 
     def short(k):
-        m = re.search(r"(dg_apply\w*kernel|conv_var\w*kernel)<[^(]*>", k)
+        m = re.search(r"(dg_apply\w*kernel|dg_mfma_kernel|conv_var\w*kernel)<[^(]*>", k)
         return m.group(0) if m else None
 
     out = ["| kernel | workload | us | HBM frac | VALU busy | FP64 util | LDS busy | LDS conflict | SALU busy "
@@ -606,8 +606,9 @@ def main():
                    "cells": n ** 3, "degree": k, "dofs": N},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(n, k),
-                     "kernel": (f"dg_apply_rowreg_kernel<{k + 1},double,...>" if n % {1: 64, 2: 32, 3: 16}[k] == 0
-                                else f"dg_apply_kernel<{k + 1},double,...>"), "kernel_avg_us": kern_ms * 1e3,
+                     "kernel": (f"dg_mfma_kernel<{k + 1},...>" if k >= 2 else
+                                "dg_apply_rowreg_kernel<2,double,...>" if n % 64 == 0 else
+                                "dg_apply_kernel<2,double,...>"), "kernel_avg_us": kern_ms * 1e3,
                      "burst_kernel_avg_us": burst_ms * 1e3, "burst_frac": alg_bytes / (burst_ms * 1e-3) / 1e9 / 8000.0,
                      "algorithmic_bytes_per_launch": alg_bytes,
                      "fp32_kernel_avg_us": kern32_ms * 1e3,
@@ -618,7 +619,7 @@ def main():
     }
     if variants:
         q2 = variants["q2_96_constant_kappa"]
-        out["roofline_q2"] = {"bound": "hbm", "kernel": "dg_apply_rowreg_kernel<3,double,...>",
+        out["roofline_q2"] = {"bound": "hbm", "kernel": "dg_mfma_kernel<3,...>",
                               "workload": "96^3 Q2 SIPG, constant kappa, FP64 y = J z",
                               "achieved": q2["fp64_GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                               "frac": q2["fp64_frac"], "kernel_avg_us": q2["fp64_us"],

@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -13,6 +15,7 @@
 #include "block_jacobi.hh"
 #include "dg_kernels.hh"
 #include "dg_load.hh"
+#include "dg_mfma.hh"
 #include "dg_tables.hh"
 #include "dg_velocity.hh"
 #include "output.hh"
@@ -32,6 +35,14 @@ struct BlockJacobiData {
   float* rm32 = nullptr;
 };
 
+// Constants of the apply kernels on the device, one allocation.
+struct DeviceTables {
+  // constant-coefficient line matrices: [0] J, [1] J^T
+  LineMats<double> lm64[2];
+  LineMats<float> lm32[2];
+  MfmaTab mfma[4];  // matrix-core apply: J, J^T, then their convection parts (cell-wise kappa)
+};
+
 struct pdelab_gpu_gridoperator {
   pdelab_config cfg;
   int device = 0;
@@ -49,6 +60,7 @@ struct pdelab_gpu_gridoperator {
   float* d_kappa32 = nullptr;
   double* d_fc64 = nullptr;  // per-cell face coefficients (FC values per cell) of kappa
   float* d_fc32 = nullptr;
+  double* d_fw64 = nullptr;  // per-cell kappa and face weights of the matrix-core apply
   double* d_R0 = nullptr;
   bool R0_valid = false;
   double* d_src = nullptr;
@@ -73,9 +85,8 @@ struct pdelab_gpu_gridoperator {
   int* h_state = nullptr;        // pinned mirrors
   double* h_dstate = nullptr;
   double* d_bscal = nullptr;     // device BiCGSTAB loop: {rho, rho_new, alpha, omega, beta}
-  // constant-coefficient line matrices: [0] J, [1] J^T
-  LineMats<double>* d_lm64 = nullptr;
-  LineMats<float>* d_lm32 = nullptr;
+  DeviceTables* d_tab = nullptr;  // constants of the apply kernels
+  MfmaX mfma_x[4];
   bool sym[2] = {false, false};  // J / J^T have the structure of line_op_sym
   // apply kernel: 0 the row kernel (x-row chunks), 1 the general kernel (chunks of consecutive cells)
   int apply_variant = 0;
@@ -133,8 +144,8 @@ inline long long apply_cpb(const H* h) {
   return h->n1 == 2 ? ApplyShape<2>::CPB : (h->n1 == 3 ? ApplyShape<3>::CPB : ApplyShape<4>::CPB);
 }
 
-// Whether an apply launch takes the row kernel (chunks of x-rows) rather than the general
-// kernel (chunks of consecutive cells). Rows that split into whole chunks always do. The
+// Whether an apply launch in FP32, or of Q1, takes the row kernel (chunks of x-rows) rather than
+// the general kernel (chunks of consecutive cells). Rows that split into whole chunks always do. The
 // partial last chunk of a row is moved back to overlap the previous one (nx > CPB), and
 // its overlapping lanes do work that is not stored, so such grids take the row kernel only
 // for the constant-coefficient symmetric operator, where it is fastest (0.78 of the
@@ -170,6 +181,43 @@ inline int apply_walk(const H* h) {
   return 1;
 }
 
+// Whether an FP64 apply takes the matrix-core kernel (dg_mfma.hh): Q2 and Q3, planes of at
+// least four cells (a wave's group) whose byte offsets stay below 4 GiB. It is faster than the
+// row and general kernels on every grid measured (row or general kernel -> this one, three
+// states in turn): 64^3 Q3 78.6 -> 61.6 us, convection 105.5 -> 66.3, lognormal kappa 117.5 ->
+// 71.7; 96^3 Q2 145.1 -> 116.6, 204.2 -> 128.9, 265.0 -> 160.2; 83x61x71 Q2 lognormal 116.8 ->
+// 65.6; 100^3 Q3 337.5 -> 258.7; 32^3 Q2 7.5 -> 5.0; 24^3 Q3 5.8 -> 4.5. A Q1 cell would fill an
+// eighth of the 4x4x4 blocks.
+inline bool mfma_kernel(const H* h) {
+  const long long np = (long long)h->a64.n[0] * h->a64.n[1];
+  return h->apply_variant == 0 && h->n1 >= 3 && np >= 4 && np * h->nloc * 8 < (1LL << 32);
+}
+
+// One launch of the matrix-core apply: workgroups of four waves of four cells cover a plane,
+// zsegs of them a column. A wave's start (its first planes and constants) costs about two
+// steps, so walks are long: up to 32 steps, 8 or more where that still gives 1024 workgroups
+// (four waves per SIMD), and shorter only for 512 workgroups. Walks of 4 / 8 / 16 / 32 steps:
+// 64^3 Q3 72 / 63 / 62 / 61 us, 64^3 Q2 - / 34.2 / 33.8 / 36.9 us; of 1 / 2 / 4: 32^3 Q2 7.5 / 7.0 /
+// 6.9 us.
+struct MfmaGrid {
+  long long wgs;  // workgroups of a plane
+  int zsegs, zw;
+};
+inline MfmaGrid mfma_grid(const H* h) {
+  const long long np = (long long)h->a64.n[0] * h->a64.n[1], nz = h->a64.n[2];
+  MfmaGrid g;
+  g.wgs = (np + 15) / 16;
+  auto cover = [&](long long target) { return (target + g.wgs - 1) / g.wgs; };
+  const long long segs = std::max({(nz + 31) / 32, std::min(cover(1024), (nz + 7) / 8), std::min(cover(512), nz)});
+  g.zw = (int)((nz + segs - 1) / segs);
+  g.zsegs = (int)((nz + g.zw - 1) / g.zw);
+  return g;
+}
+inline long long mfma_blocks(const H* h) {
+  const MfmaGrid g = mfma_grid(h);
+  return g.wgs * g.zsegs;
+}
+
 inline int fail(H* h, int code, const std::string& msg) {
   if (h) h->err = msg;
   return code;
@@ -197,15 +245,22 @@ inline const DGArgs<float>& args_for<float>(H* h) { return h->a32; }
 template <typename T>
 inline const LineMats<T>* line_mats(H* h, bool trans);
 template <>
-inline const LineMats<double>* line_mats<double>(H* h, bool trans) { return h->d_lm64 + (trans ? 1 : 0); }
+inline const LineMats<double>* line_mats<double>(H* h, bool trans) { return h->d_tab->lm64 + (trans ? 1 : 0); }
 template <>
-inline const LineMats<float>* line_mats<float>(H* h, bool trans) { return h->d_lm32 + (trans ? 1 : 0); }
+inline const LineMats<float>* line_mats<float>(H* h, bool trans) { return h->d_tab->lm32 + (trans ? 1 : 0); }
 
 // y (+)= J z (or J^T z) on the handle's stream for Q_{N1-1}: mode 0 y = J z, 1 y += J z,
 // 2 y = J z with the fused z.(Jz) partials in dotp. Defined in apply_q<N1-1>.hip.
 template <int N1, typename T>
 int launch_apply_n(H* h, const T* z, T* y, const T* fc, const DGArgs<T>& a, bool trans, int mode, T* dotp,
                    const int* stop);
+
+// The FP64 apply on the matrix cores (apply_mfma.hip; modes as above) and its constants, from
+// the 1D matrices of J and J^T without reaction and their convection parts.
+int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop);
+void mfma_setup(H* h, const DGArgs<long double>& al, const LineMats<long double> (&m)[2],
+                const LineMats<long double> (&mconv)[2], MfmaTab (&t)[4]);
+int mfma_weights(H* h);  // d_fw64 from the current face coefficients
 
 // Block Jacobi (block_jacobi.hip): data set-up for the given precision (64 or 32),
 // invalidation when kappa changes, the launches (BJ_PREC / BJ_ADD / BJ_CGR, see

@@ -220,17 +220,34 @@ static bool symmetric_form(const DGArgs<LD>& al, const LineMats<LD>& m, int n, L
   return true;
 }
 
+static bool build_line_mats_pair(const DGArgs<LD>& al, int n1, LineMats<LD> (&m)[2]) {
+  switch (n1) {
+    case 2: return build_line_mats_n<2, false>(al, m[0]) && build_line_mats_n<2, true>(al, m[1]);
+    case 3: return build_line_mats_n<3, false>(al, m[0]) && build_line_mats_n<3, true>(al, m[1]);
+    default: return build_line_mats_n<4, false>(al, m[0]) && build_line_mats_n<4, true>(al, m[1]);
+  }
+}
+
+// Constants of the matrix-core apply: the line matrices without reaction, and the
+// convection part alone (S = 0), which cell-wise kappa adds to its own combination.
+static int build_mfma(H* h, MfmaTab (&t)[4]) {
+  DGArgs<LD> al;
+  fill_args<LD>(h, al);
+  al.c = al.vc = 0;
+  DGArgs<LD> ac = al;
+  for (int d = 0; d < 3; ++d) ac.S[d] = 0;
+  LineMats<LD> m[2], mc[2];
+  if (!build_line_mats_pair(al, h->n1, m) || !build_line_mats_pair(ac, h->n1, mc))
+    return fail(h, PDELAB_ERR_INVALID_ARG, "constant-coefficient line operator is not of rank-two face form");
+  mfma_setup(h, al, m, mc, t);
+  return PDELAB_OK;
+}
+
 static int build_line_mats(H* h) {
   DGArgs<LD> al;
   fill_args<LD>(h, al);
   LineMats<LD> m[2];
-  bool ok = true;
-  switch (h->n1) {
-    case 2: ok = build_line_mats_n<2, false>(al, m[0]) && build_line_mats_n<2, true>(al, m[1]); break;
-    case 3: ok = build_line_mats_n<3, false>(al, m[0]) && build_line_mats_n<3, true>(al, m[1]); break;
-    default: ok = build_line_mats_n<4, false>(al, m[0]) && build_line_mats_n<4, true>(al, m[1]); break;
-  }
-  if (!ok) return fail(h, PDELAB_ERR_INVALID_ARG, "constant-coefficient line operator is not of rank-two face form");
+  if (!build_line_mats_pair(al, h->n1, m)) return fail(h, PDELAB_ERR_INVALID_ARG, "constant-coefficient line operator is not of rank-two face form");
   for (int t = 0; t < 2; ++t) {
     LD Ah[4][4], Ph[4], Qh[4];
     h->sym[t] = symmetric_form(al, m[t], h->n1, Ah, Ph, Qh);
@@ -245,13 +262,12 @@ static int build_line_mats(H* h) {
       }
     }
   }
-  LineMats<double> m64[2];
-  LineMats<float> m32[2];
-  for (int t = 0; t < 2; ++t) { cast_line_mats(m[t], m64[t]); cast_line_mats(m[t], m32[t]); }
-  HIPCHK(h, hipMalloc(&h->d_lm64, sizeof(m64)));
-  HIPCHK(h, hipMalloc(&h->d_lm32, sizeof(m32)));
-  HIPCHK(h, hipMemcpy(h->d_lm64, m64, sizeof(m64), hipMemcpyHostToDevice));
-  HIPCHK(h, hipMemcpy(h->d_lm32, m32, sizeof(m32), hipMemcpyHostToDevice));
+  DeviceTables tabs;
+  std::memset(&tabs, 0, sizeof(tabs));
+  for (int t = 0; t < 2; ++t) { cast_line_mats(m[t], tabs.lm64[t]); cast_line_mats(m[t], tabs.lm32[t]); }
+  if (h->n1 >= 3) CHK(build_mfma(h, tabs.mfma));
+  HIPCHK(h, hipMalloc(&h->d_tab, sizeof(tabs)));
+  HIPCHK(h, hipMemcpy(h->d_tab, &tabs, sizeof(tabs), hipMemcpyHostToDevice));
   return PDELAB_OK;
 }
 
@@ -328,6 +344,12 @@ static int apply_mode(H* h, const T* z, T* y, bool trans, int mode, T* dotp = nu
   CHK(check_outflow(h));
   if (h->varb && mode == 2)
     return fail(h, PDELAB_ERR_UNSUPPORTED, "velocity field: CG (non-symmetric operator), use BiCGSTAB");
+  if constexpr (std::is_same<T, double>::value) {
+    if (mfma_kernel(h)) {
+      CHK(launch_apply_mfma(h, z, y, trans, mode, dotp, stop));
+      return vel_launch<T>(h, z, y, stop, trans);
+    }
+  }
   int st = PDELAB_ERR_UNSUPPORTED;
   switch (h->n1) {
     case 2: st = launch_apply_n<2, T>(h, z, y, fc_for<T>(h), args_for<T>(h), trans, mode, dotp, stop); break;
@@ -348,12 +370,16 @@ template <typename T>
 static int apply_t(H* h, const T* z, T* y, bool trans, bool accum) {
   return apply_mode<T>(h, z, y, trans, accum ? 1 : 0);
 }
-// partials of the fused apply dot: one per apply workgroup (a walking workgroup covers
-// apply_walk(h) chunks)
-static long long apply_partials(H* h) { return apply_blocks(h) / apply_walk(h); }
+// partials of the fused apply dot: one per apply workgroup (a walking workgroup of the row
+// kernel covers apply_walk(h) chunks)
+template <typename T>
+static long long apply_partials(H* h) {
+  if (sizeof(T) == 8 && h->n1 >= 3) return mfma_kernel(h) ? mfma_blocks(h) : apply_blocks_of(h, false);
+  return apply_blocks(h) / apply_walk(h);
+}
 
 // PDELAB_GPU_APPLY=general runs the general apply kernel on every grid (for comparison;
-// by default row_kernel() chooses per launch).
+// by default mfma_kernel() and row_kernel() choose per launch).
 static void choose_apply_shape(H* h) {
   const char* v = std::getenv("PDELAB_GPU_APPLY");
   h->apply_variant = (v && std::strcmp(v, "general") == 0) ? 1 : 0;
@@ -594,10 +620,10 @@ template <typename T, typename A>
 static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool trans, int maxit, double def_ref,
                    double red, CgLoopOut& out) {
   const long long n = h->N;
-  const long long nbapply = apply_partials(h);
-  // sized for either kernel: the choice can change with set_kappa
+  const long long nbapply = apply_partials<T>(h);
+  // sized for every kernel: the choice can change with set_kappa and with the precision
   if (!h->d_applydot) {
-    const long long nmax = std::max(std::max(apply_blocks_of(h, true), apply_blocks_of(h, false)), 1LL);
+    const long long nmax = std::max({apply_blocks_of(h, true), apply_blocks_of(h, false), mfma_blocks(h), 1LL});
     HIPCHK(h, hipMalloc(&h->d_applydot, sizeof(double) * (size_t)nmax));
   }
   static_assert(std::is_same<T, A>::value, "the fused apply dot is accumulated in the vector type");
@@ -865,7 +891,11 @@ static int validate(const pdelab_config* c, std::string& msg) {
 // per-cell face coefficients of the current kappa (FP64 and FP32) for the apply kernels
 static int update_face_coeffs(H* h) {
   const long long nc = h->ncells;
-  if (!h->d_fc64) HIPCHK(h, hipMalloc(&h->d_fc64, sizeof(double) * FC * nc));
+  if (!h->d_fc64) {  // with the rows of the matrix-core apply behind
+    const int row = h->n1 >= 3 ? mfma_row(h->a64.aniso) : 0;
+    HIPCHK(h, hipMalloc(&h->d_fc64, sizeof(double) * (FC + row) * nc));
+    h->d_fw64 = h->d_fc64 + FC * nc;
+  }
   if (!h->d_fc32) HIPCHK(h, hipMalloc(&h->d_fc32, sizeof(float) * FC * nc));
   const int nb = (int)((nc + 255) / 256);
   hipLaunchKernelGGL(face_coeff_kernel<double>, dim3(nb), dim3(256), 0, h->stream, (const double*)h->d_kappa,
@@ -873,6 +903,7 @@ static int update_face_coeffs(H* h) {
   hipLaunchKernelGGL(face_coeff_kernel<float>, dim3(nb), dim3(256), 0, h->stream, (const double*)h->d_kappa,
                      h->d_fc32, h->a64);
   HIPCHK(h, hipGetLastError());
+  if (h->n1 >= 3) CHK(mfma_weights(h));
   bj_invalidate(h);
   return PDELAB_OK;
 }
@@ -1378,7 +1409,7 @@ int pdelab_gpu_destroy(pdelab_gpu_gridoperator* h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   void* ptrs[] = {h->d_kappa, h->d_kappa32, h->d_R0, h->d_src, h->d_ftab, h->d_gtab, h->d_diag, h->d_dinv,
                   h->d_dinv32, h->d_part64, h->d_part32, h->d_scal64, h->d_scal32, h->d_applydot,
-                  h->d_state, h->d_dstate, h->d_bscal, h->d_lm64, h->d_lm32, h->d_fc64, h->d_fc32};
+                  h->d_state, h->d_dstate, h->d_bscal, h->d_tab, h->d_fc64, h->d_fc32};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (double* p : h->os)
