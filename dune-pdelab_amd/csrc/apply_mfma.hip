@@ -25,8 +25,10 @@ static void launch_kind(H* h, const double* z, double* y, const MfmaTab* tab, co
   else launch_mode<N1, MFMA_WEIGHT>(h, z, y, tab, a, nb, mode, dotp, stop);
 }
 
-int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop) {
+// Arguments of one launch without the field's.
+MfmaArgs mfma_args(const H* h, bool trans) {
   MfmaArgs a;
+  std::memset(&a, 0, sizeof(a));
   const DGArgs<double>& d = h->a64;
   a.nx = d.n[0];
   a.ny = d.n[1];
@@ -45,7 +47,12 @@ int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, do
   a.x = h->mfma_x[(trans ? 1 : 0) + (h->vark ? 2 : 0)];
   if (!h->vark)
     for (int i = 0; i < h->n1; ++i) a.x.A[i][i] += a.vc;
-  const unsigned nb = (unsigned)(grid.wgs * grid.zsegs);
+  return a;
+}
+
+int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop) {
+  const MfmaArgs a = mfma_args(h, trans);
+  const unsigned nb = (unsigned)mfma_blocks(h);
   // J and J^T, each with the whole matrices and with their convection part (cell-wise kappa)
   const MfmaTab* tab = h->d_tab->mfma + (trans ? 1 : 0) + (h->vark ? 2 : 0);
   if (h->n1 == 3) launch_kind<3>(h, z, y, tab, a, nb, mode, dotp, stop);

@@ -27,6 +27,10 @@
 // 4.4 TB/s; reads 1.17x and writes 1.0x the algorithmic bytes; without memory traffic 31 us, so
 // it is bound by HBM and its latency), lognormal kappa 117 -> 72 us; 96^3 Q2 145 -> 118 us (70 us
 // without memory traffic: 9/16 of the matrix lanes are padding), convection 204 -> 129 us.
+// With a velocity field (before: the apply with b = 0, then a kernel of one cell per wave and
+// seven barrier phases over LDS): 64^3 Q2 296 -> 107 us (340 MB, 3.2 TB/s), 40^3 Q3 145 -> 46 us, with
+// cell-wise kappa 141 -> 66 us. Two waves per SIMD hold 170 to 256 registers; three spill and
+// were slower (112 us). Bound by the latency of a step's chain of 93 (Q2) or 120 products.
 #ifndef PDELAB_DG_MFMA_HH
 #define PDELAB_DG_MFMA_HH
 
@@ -65,6 +69,14 @@ struct MfmaX {
   double d1[4], M[4][4], A[4][4], P[4], Q[4];
 };
 
+// Constants of the velocity field's terms for M points per direction. Lane matrices as above:
+// LB, LD point by node, WB = (w B)^T, WDy = vs_1 (w D)^T, WDz = vs_2 (w D)^T node by point; scalars
+// for the x-lines, indexed [point][node]: B, D, BW = w B, DW = vs_0 w D. vs = -|K| / h, area = |K| / h.
+struct MfmaVelTab {
+  double LB[16], LD[16], WB[16], WDy[16], WDz[16];
+  double B[4][4], D[4][4], BW[4][4], DW[4][4];
+};
+
 struct MfmaArgs {
   int nx, ny, nz;
   unsigned np;     // cells of a plane
@@ -75,6 +87,10 @@ struct MfmaArgs {
   double S[3], fg, fh, alphak;
   int weightsOn, bc[6];
   MfmaX x;
+  // velocity field at the quadrature points (layout of dg_velocity.hh), or null
+  const double *bv, *bf;
+  const MfmaVelTab* vt;
+  double vs[3], area[3];
 };
 
 // Constant kappa, symmetric line operator (no convection); cell-wise kappa with one weight per
@@ -219,9 +235,23 @@ __device__ __forceinline__ double dpp_block(double old, double src) {
 }
 constexpr int kPrevBlock = 0x114, kNextBlock = 0x104;
 
-// MODE 0: y = J z, 1: y += J z, 2: y = J z and partials of z . (J z), one per workgroup
-template <int N1, int KIND, int MODE>
-__global__ __launch_bounds__(256, (mfma_waves<N1, KIND>())) void dg_mfma_kernel(const double* __restrict__ z, double* __restrict__ y,
+// src of lane 2 / 3 of the quad in lanes 0 / 1 (and 2 / 3)
+__device__ __forceinline__ double dpp_upper_pair(double src) {
+  const long long s = __double_as_longlong(src);
+  const int lo = __builtin_amdgcn_mov_dpp((int)s, 0xee, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(s >> 32), 0xee, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// MODE 0: y = J z, 1: y += J z, 2: y = J z and partials of z . (J z), one per workgroup.
+// VEL 1 (J), 2 (J^T): adds the convection terms of the velocity field at M points per direction
+// (dg_velocity.hh states them). They too are 4x4x4 products: z at the points by contracting x
+// in registers, z (T0 -> T1) and y; the products with b; and the tests back, y (T1 -> T0) and z.
+// The traces of the y faces are gathered into one product, own lower / own upper / lower
+// neighbour's / upper neighbour's along lane%4 (T1 -> lane/16 = z), interpolated, upwinded with a
+// quad permutation and tested back; the z faces likewise from T0, the x faces per register.
+template <int N1, int KIND, int MODE, int VEL = 0, int M = N1>
+__global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mfma_kernel(const double* __restrict__ z, double* __restrict__ y,
                                                       const double* __restrict__ fc, const MfmaTab* __restrict__ tab,
                                                       const MfmaArgs a, unsigned nblocks, double* __restrict__ dotp,
                                                       const int* __restrict__ stop) {
@@ -375,6 +405,185 @@ __global__ __launch_bounds__(256, (mfma_waves<N1, KIND>())) void dg_mfma_kernel(
     SG::put(buf, se[0], v[0]);
     if (two) SG::put(buf, se[1], v[1]);
   };
+  // ---- velocity field
+  constexpr int M2 = M * M, M3 = M2 * M, VM = VEL ? M : 1, VN = VEL ? N1 : 1;
+  double LB = 0, LD = 0, WB = 0, WDy = 0, WDz = 0, Po = 0, Pl = 0, Pu = 0, Eo = 0, say = 0, saz = 0;
+  double b0[VM], b1[VM], b2[VM], by[VM], bz[VM], bxl = 0, bxu = 0;  // the field at this step's points
+  double tz[VN];  // the lower z-neighbour's trace part
+  unsigned ov = 0, ofx = 0, ofy = 0;
+  bool outy = false;
+  // boundary sides with a convection term
+  auto takes = [&](int side) -> int { return int(a.bc[side] == BC_DIRICHLET) | int(a.bc[side] == BC_OUTFLOW); };
+  if constexpr (VEL != 0) {
+    LB = a.vt->LB[me];
+    WB = a.vt->WB[me];
+    if constexpr (VEL == 1) {
+      WDy = a.vt->WDy[me];
+      WDz = a.vt->WDz[me];
+    } else {
+      LD = a.vt->LD[me];
+    }
+    // gather: own lower, own upper, lower neighbour's, upper neighbour's trace; scatter: its transpose
+    Po = (i4 == 0 && k4 == 0) || (i4 == 1 && k4 == N1 - 1) ? 1.0 : 0.0;
+    Pl = i4 == 2 && k4 == N1 - 1 ? 1.0 : 0.0;
+    Pu = i4 == 3 && k4 == 0 ? 1.0 : 0.0;
+    Eo = (i4 == 0 && k4 == 0) || (i4 == N1 - 1 && k4 == 1) ? 1.0 : 0.0;
+    // signed face areas of the lane's y and z face (lower, upper); zero where the face has no term
+    // (here and below as selects: hipcc 7.2 dropped the assignment of nested short-circuit branches)
+    const bool lo = i4 == 0, up = i4 == 1;
+    const double sl = (int(loy) | takes(2)) ? -a.area[1] : 0.0, su = (int(hiy) | takes(3)) ? a.area[1] : 0.0;
+    say = lo ? sl : (up ? su : 0.0);
+    outy = (lo ? int(!loy) & int(a.bc[2] == BC_OUTFLOW) : up ? int(!hiy) & int(a.bc[3] == BC_OUTFLOW) : 0) != 0;
+    saz = i4 == 0 ? -a.area[2] : (i4 == 1 ? a.area[2] : 0.0);
+    const int qi = min(i4, M - 1), qk = min(k4, M - 1);
+    ov = (cc * (3 * M3) + M * (qk + M * qi)) * 8u;              // volume, T1: lane%4 = z point, lane/16 = y point
+    ofx = (cc * (6 * M2) + qi + M * qk) * 8u;                   // x faces, T0: lane%4 = y point, lane/16 = z point
+    ofy = (cc * (6 * M2) + (2 + (i4 & 1)) * M2 + M * qk) * 8u;  // y faces: lane%4 = side; the z faces 2 M2 further
+  }
+  auto load_field = [&](int kz) {
+    if constexpr (VEL != 0) {
+      const mfma_gp bv = per_step<mfma_gp>(a.bv + (size_t)kz * a.np * (3 * M3));
+      const mfma_gp bf = per_step<mfma_gp>(a.bf + (size_t)kz * a.np * (6 * M2));
+      auto row = [&](mfma_gp base, unsigned off, double (&v)[VM]) {
+        const mfma_gp q = (mfma_gp)((const char __attribute__((address_space(1)))*)base + here(off));
+#pragma unroll
+        for (int e = 0; e < M; ++e) v[e] = q[e];
+      };
+      row(bv, ov, b0);
+      row(bv, ov + M3 * 8, b1);
+      row(bv, ov + 2 * M3 * 8, b2);
+      row(bf, ofy, by);
+      row(bf, ofy + 2 * M2 * 8, bz);
+      const mfma_gp q = (mfma_gp)((const char __attribute__((address_space(1)))*)bf + here(ofx));
+      bxl = q[0];
+      bxu = q[M2];
+    }
+  };
+  // upwinded flux of a face point: sa the signed area (the weights come with the test)
+  auto flux = [&](double own, double nb, double b, double sa, bool out) {
+    const double cf = sa * b;
+    const bool in = (int(out) | int(cf >= 0.0)) != 0;
+    if constexpr (VEL == 2) return in ? cf * (out ? own : own - nb) : 0.0;
+    return cf * (in ? own : nb);
+  };
+  // o (T0) += the convection terms of the step's cells: own lines uz (T0) and u (T1), the upper
+  // plane's zr (T0), the x-neighbours' traces vl, vr (T1)
+  auto convect = [&](int kz, const double (&uz)[N1], const double (&zr)[N1], const double (&u)[N1], double vl, double vr,
+                     double (&o)[N1]) {
+    if constexpr (VEL != 0) {
+      typedef const MfmaVelTab __attribute__((address_space(4))) * tp;
+      const bool loz = kz > 0, hiz = kz < a.nz - 1;
+      // x faces
+      {
+        const double ol = mfma4(LB, mfma4(u[0], LB, 0.0), 0.0), ou = mfma4(LB, mfma4(u[N1 - 1], LB, 0.0), 0.0);
+        const double nl = mfma4(LB, mfma4(vl, LB, 0.0), 0.0), nu = mfma4(LB, mfma4(vr, LB, 0.0), 0.0);
+        const double sl = (int(lox) | takes(0)) ? -a.area[0] : 0.0, su = (int(hix) | takes(1)) ? a.area[0] : 0.0;
+        const double fl = flux(ol, nl, bxl, sl, (int(!lox) & int(a.bc[0] == BC_OUTFLOW)) != 0);
+        const double fu = flux(ou, nu, bxu, su, (int(!hix) & int(a.bc[1] == BC_OUTFLOW)) != 0);
+        o[0] = mfma4(mfma4(fl, WB, 0.0), WB, o[0]);
+        o[N1 - 1] = mfma4(mfma4(fu, WB, 0.0), WB, o[N1 - 1]);
+      }
+      // gathered traces t[x] (lane%4 = side, lane/16 = the other direction): the points, the flux,
+      // the test along x and that direction; returns g[x] (lane%4 = the other direction, lane/16 = side)
+      auto face = [&](const double (&t)[N1], const double (&b)[VM], double sa, bool out, double (&g)[N1]) {
+        const tp v = per_step<tp>(a.vt);
+        double f[VM];
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+          double w = 0;
+#pragma unroll
+          for (int e = 0; e < N1; ++e) w += v->B[q][e] * t[e];
+          w = mfma4(LB, w, 0.0);
+          f[q] = flux(w, dpp_upper_pair(w), b[q], sa, out);
+        }
+#pragma unroll
+        for (int e = 0; e < N1; ++e) {
+          double w = 0;
+#pragma unroll
+          for (int q = 0; q < M; ++q) w += v->BW[q][e] * f[q];
+          g[e] = mfma4(w, WB, 0.0);
+        }
+      };
+      {
+        double t[N1], g[N1], n[N1];
+        SG::line(BYL, a1, n);
+#pragma unroll
+        for (int e = 0; e < N1; ++e) t[e] = mfma4(n[e], loy ? Pl : 0.0, mfma4(u[e], Po, 0.0));
+        SG::line(BYR, a1, n);
+#pragma unroll
+        for (int e = 0; e < N1; ++e) t[e] = mfma4(n[e], hiy ? Pu : 0.0, t[e]);
+        face(t, by, say, outy, g);
+#pragma unroll
+        for (int e = 0; e < N1; ++e) o[e] = mfma4(g[e], Eo, o[e]);
+      }
+      {
+        double t[N1], g[N1];
+        const double pu = hiz ? Pu : 0.0;
+#pragma unroll
+        for (int e = 0; e < N1; ++e) {
+          t[e] = mfma4(zr[e], pu, mfma4(uz[e], Po, tz[e]));
+          tz[e] = mfma4(uz[e], Pl, 0.0);
+        }
+        const int lo = int(i4 == 0) & int(!loz), up = int(i4 == 1) & int(!hiz);
+        const double sa = (lo & (1 - takes(4))) | (up & (1 - takes(5))) ? 0.0 : saz;
+        const bool out = ((lo & int(a.bc[4] == BC_OUTFLOW)) | (up & int(a.bc[5] == BC_OUTFLOW))) != 0;
+        face(t, bz, sa, out, g);
+#pragma unroll
+        for (int e = 0; e < N1; ++e) o[e] = mfma4(Eo, g[e], o[e]);
+      }
+      // volume
+      const tp v = per_step<tp>(a.vt);
+      if constexpr (VEL == 1) {
+        double p0[VM], p1[VM], p2[VM];
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+          double w = 0;
+#pragma unroll
+          for (int e = 0; e < N1; ++e) w += v->B[q][e] * uz[e];
+          w = mfma4(LB, mfma4(w, LB, 0.0), 0.0);
+          p0[q] = b0[q] * w;
+          p1[q] = b1[q] * w;
+          p2[q] = b2[q] * w;
+        }
+        const tp r = per_step<tp>(a.vt);
+#pragma unroll
+        for (int e = 0; e < N1; ++e) {
+          double w0 = 0, w1 = 0, w2 = 0;
+#pragma unroll
+          for (int q = 0; q < M; ++q) {
+            w0 += r->DW[q][e] * p0[q];
+            w1 += r->BW[q][e] * p1[q];
+            w2 += r->BW[q][e] * p2[q];
+          }
+          const double tB = mfma4(w1, WDy, mfma4(w0, WB, 0.0)), tD = mfma4(w2, WB, 0.0);
+          o[e] = mfma4(WDz, tD, mfma4(WB, tB, o[e]));
+        }
+      } else {
+        double p[VM];
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+          double w = 0, d = 0;
+#pragma unroll
+          for (int e = 0; e < N1; ++e) {
+            w += v->B[q][e] * uz[e];
+            d += v->D[q][e] * uz[e];
+          }
+          const double zB = mfma4(w, LB, 0.0);
+          const double gx = mfma4(LB, mfma4(d, LB, 0.0), 0.0), gy = mfma4(LD, zB, 0.0);
+          const double gz = mfma4(LB, mfma4(w, LD, 0.0), 0.0);
+          p[q] = a.vs[0] * b0[q] * gx + a.vs[1] * b1[q] * gy + a.vs[2] * b2[q] * gz;
+        }
+        const tp r = per_step<tp>(a.vt);
+#pragma unroll
+        for (int e = 0; e < N1; ++e) {
+          double w = 0;
+#pragma unroll
+          for (int q = 0; q < M; ++q) w += r->BW[q][e] * p[q];
+          o[e] = mfma4(WB, mfma4(w, WB, 0.0), o[e]);
+        }
+      }
+    }
+  };
   double ua[N1], ub[N1], sn[N1];  // own T0 lines of even / odd steps, lower z-neighbour's part of s
   double wz = 0;                  // face weights: that of the lower z face
   {
@@ -391,6 +600,10 @@ __global__ __launch_bounds__(256, (mfma_waves<N1, KIND>())) void dg_mfma_kernel(
   SG::line(W, a0, ua);
 #pragma unroll
   for (int e = 0; e < N1; ++e) sn[e] = 0;
+  if constexpr (VEL != 0) {
+#pragma unroll
+    for (int e = 0; e < N1; ++e) tz[e] = 0;
+  }
   if (k0 > 0) {
     double zl[N1], Nl = Nzl;
     SG::line(BYL, a0, zl);
@@ -398,6 +611,10 @@ __global__ __launch_bounds__(256, (mfma_waves<N1, KIND>())) void dg_mfma_kernel(
     if constexpr (KIND == MFMA_GENERAL) Nl = lower_z(k0);
 #pragma unroll
     for (int e = 0; e < N1; ++e) sn[e] = mfma4(zl[e], Nl, 0.0);
+    if constexpr (VEL != 0) {
+#pragma unroll
+      for (int e = 0; e < N1; ++e) tz[e] = mfma4(zl[e], Pl, 0.0);
+    }
   }
   // entry (i, j) of a centro-symmetric matrix, read at the lexicographically first position
   auto centro = [](const double(&m)[4][4], int i, int j) {
@@ -408,6 +625,7 @@ __global__ __launch_bounds__(256, (mfma_waves<N1, KIND>())) void dg_mfma_kernel(
   // one z-step: own cells in B0 (T0 lines uz), the next plane's to B1 (T0 lines zr)
   auto step = [&](int kz, double* B0, double* B1, double (&uz)[N1], double (&zr)[N1]) {
     const bool loz = kz > 0, hiz = kz < a.nz - 1;
+    load_field(kz);  // older than the next step's loads: waited for without them
     wave_lds_fence();
     put(B1, rn);
     put(BYL, rl);
@@ -624,6 +842,7 @@ __global__ __launch_bounds__(256, (mfma_waves<N1, KIND>())) void dg_mfma_kernel(
     }
 #pragma unroll
     for (int i = 0; i < N1; ++i) o[i] = mfma4(Mm, o[i], 0.0);
+    convect(kz, uz, zr, u, vl, vr, o);
     if constexpr (MODE == 2) {  // the own lines again, from LDS: held through the step they would spill
       double v[N1];
       SG::line(B0, a0, v);
@@ -648,13 +867,13 @@ __global__ __launch_bounds__(256, (mfma_waves<N1, KIND>())) void dg_mfma_kernel(
       }
     }
   };
-  double *const WB = W + SG::BUF;
+  double* const W1 = W + SG::BUF;
   int kz = k0;
   for (; kz + 1 < k1; kz += 2) {
-    step(kz, W, WB, ua, ub);
-    step(kz + 1, WB, W, ub, ua);
+    step(kz, W, W1, ua, ub);
+    step(kz + 1, W1, W, ub, ua);
   }
-  if (kz < k1) step(kz, W, WB, ua, ub);
+  if (kz < k1) step(kz, W, W1, ua, ub);
   if constexpr (MODE == 2) {
     double v[1] = {pq};
     block_sum_reuse<4, double, 1>(v, lds);

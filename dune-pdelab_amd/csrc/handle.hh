@@ -119,6 +119,7 @@ struct pdelab_gpu_gridoperator {
   VelArgs<double> va64;
   VelArgs<float> va32;
   VelArgs<double>* d_va64 = nullptr;  // device copy for the cell-block set-up
+  MfmaVelTab* d_mfma_vel = nullptr;   // constants of the matrix-core apply with the field
   double* d_sortmp64 = nullptr;       // block SOR with a field: the right-hand side less the couplings
   float* d_sortmp32 = nullptr;
 };
@@ -193,6 +194,13 @@ inline bool mfma_kernel(const H* h) {
   return h->apply_variant == 0 && h->n1 >= 3 && np >= 4 && np * h->nloc * 8 < (1LL << 32);
 }
 
+// Whether its velocity-field form applies: up to four points per direction (Q2 with intorderadd
+// 0..3, Q3 with 0 or 1), the field's in-plane byte offsets below 4 GiB.
+inline bool mfma_vel_kernel(const H* h) {
+  const long long np = (long long)h->a64.n[0] * h->a64.n[1], m = h->tab.m;
+  return mfma_kernel(h) && m <= 4 && (h->vark || (h->sym[0] && h->sym[1])) && np * 6 * m * m * m * 8 < (1LL << 32);
+}
+
 // One launch of the matrix-core apply: workgroups of four waves of four cells cover a plane,
 // zsegs of them a column. A wave's start (its first planes and constants) costs about two
 // steps, so walks are long: up to 32 steps, 8 or more where that still gives 1024 workgroups
@@ -260,6 +268,10 @@ int launch_apply_n(H* h, const T* z, T* y, const T* fc, const DGArgs<T>& a, bool
 int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop);
 void mfma_setup(H* h, const DGArgs<long double>& al, const LineMats<long double> (&m)[2],
                 const LineMats<long double> (&mconv)[2], MfmaTab (&t)[4]);
+MfmaArgs mfma_args(const H* h, bool trans);
+// The same with the velocity field's terms (apply_mfma_vel.hip), and their constants.
+int launch_apply_mfma_vel(H* h, const double* z, double* y, bool trans, bool accum, const int* stop);
+int mfma_vel_setup(H* h);
 int mfma_weights(H* h);  // d_fw64 from the current face coefficients
 
 // Block Jacobi (block_jacobi.hip): data set-up for the given precision (64 or 32),

@@ -345,6 +345,7 @@ static int apply_mode(H* h, const T* z, T* y, bool trans, int mode, T* dotp = nu
   if (h->varb && mode == 2)
     return fail(h, PDELAB_ERR_UNSUPPORTED, "velocity field: CG (non-symmetric operator), use BiCGSTAB");
   if constexpr (std::is_same<T, double>::value) {
+    if (h->varb && mfma_vel_kernel(h)) return launch_apply_mfma_vel(h, z, y, trans, mode == 1, stop);
     if (mfma_kernel(h)) {
       CHK(launch_apply_mfma(h, z, y, trans, mode, dotp, stop));
       return vel_launch<T>(h, z, y, stop, trans);

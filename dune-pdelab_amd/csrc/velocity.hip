@@ -33,12 +33,13 @@ static void fill_vel_args(const H* h, VelArgs<T>& a) {
 }
 
 void vel_free(H* h) {
-  void* p[] = {h->d_bv64, h->d_bf64, h->d_bv32, h->d_bf32, h->d_va64, h->d_sortmp64, h->d_sortmp32};
+  void* p[] = {h->d_bv64, h->d_bf64, h->d_bv32, h->d_bf32, h->d_va64, h->d_mfma_vel, h->d_sortmp64, h->d_sortmp32};
   for (void* q : p)
     if (q) (void)hipFree(q);
   h->d_bv64 = h->d_bf64 = nullptr;
   h->d_bv32 = h->d_bf32 = nullptr;
   h->d_va64 = nullptr;
+  h->d_mfma_vel = nullptr;
   h->d_sortmp64 = nullptr;
   h->d_sortmp32 = nullptr;
   h->varb = false;
@@ -118,6 +119,7 @@ int vel_set(H* h, const double* bvol, const double* bface) {
   fill_vel_args<float>(h, h->va32);
   HIPCHK(h, hipMalloc(&h->d_va64, sizeof(VelArgs<double>)));
   HIPCHK(h, hipMemcpy(h->d_va64, &h->va64, sizeof(VelArgs<double>), hipMemcpyHostToDevice));
+  CHK(mfma_vel_setup(h));
   h->varb = true;
   h->R0_valid = false;
   h->diag_valid = false;

@@ -80,3 +80,47 @@ def test_mfma_apply_nan_stays_local(pkg):
     go.operator_apply(go.vector(z), y)
     bad = np.flatnonzero(np.isnan(y.download().reshape(-1, 64)).any(axis=1))
     assert set(bad) <= {c, c - 1, c + 1, c - 6, c + 6, c - 24, c + 24} and c in bad
+
+
+FIELDS = {
+    "const": dict(),
+    "intorderadd2": dict(intorderadd=2),
+    "cells": dict(kappa_per_cell=1, c=0.3),
+    "cells_neumann": dict(kappa_per_cell=1, bctype=(-1, 0, -3, -1, 0, -1), method=0),
+    "cells_off": dict(kappa_per_cell=1, weights=1),
+    "tensor_add2": dict(kappa_per_cell=2, lx=2.0, ly=0.5, intorderadd=2),
+    "outflow": dict(kappa0=0.1, bctype=(0, -2, -1, 0, 0, -2)),
+}
+
+
+@pytest.mark.parametrize("degree", [2, 3])
+@pytest.mark.parametrize("kind", FIELDS)
+@pytest.mark.parametrize("grid", [(4, 1, 1), (2, 2, 3), (5, 3, 2), (3, 3, 4), (17, 1, 2), (6, 7, 34)],
+                         ids=lambda g: "x".join(map(str, g)))
+def test_mfma_velocity_edges(pkg, of, grid, kind, degree):
+    """The velocity field's terms in the same pass, J and J^T: random values (positive where a
+    side is an outflow side), so every face point's upwind choice is its own."""
+    print(f"[gpu] matrix-core apply with a velocity field {grid} Q{degree} {kind}", flush=True)
+    nx, ny, nz = grid
+    cfg = pkg.make_config(nx=nx, ny=ny, nz=nz, degree=degree, alpha=3.0, **FIELDS[kind])
+    rng = np.random.default_rng(9)
+    kappa = np.exp(rng.normal(size=pkg.ncells(cfg) * (3 if cfg.kappa_per_cell == 2 else 1))) if cfg.kappa_per_cell else None
+    m = pkg.quadrature_points(cfg)
+    nf = (nx + 1) * ny * nz + nx * (ny + 1) * nz + nx * ny * (nz + 1)
+    bv, bf = rng.normal(size=nx * ny * nz * 3 * m ** 3), rng.normal(size=nf * m ** 2)
+    if kind == "outflow":
+        bf = np.abs(bf)
+    go, o = pkg.GridOperator(cfg, kappa), of.Oracle(cfg, kappa)
+    go.set_velocity_field(bv, bf)
+    o.set_velocity_field(bv, bf)
+    z, y0 = rng.uniform(-1, 1, go.N), rng.uniform(-1, 1, go.N)
+    zd, yd = go.vector(z), go.vector(y0)
+    ref = o.jacobian_apply(z)
+    go.jacobian_apply(zd, yd)
+    assert np.linalg.norm(yd.download() - y0 - ref) <= RTOL * (np.linalg.norm(ref) + np.linalg.norm(y0))
+    go.operator_apply(zd, yd)
+    assert np.linalg.norm(yd.download() - ref) <= RTOL * np.linalg.norm(ref)
+    ref = o.jacobian_apply_transpose(z)
+    yd.zero()
+    go.jacobian_apply_transpose(zd, yd)
+    assert np.linalg.norm(yd.download() - ref) <= RTOL * np.linalg.norm(ref)
