@@ -3,26 +3,31 @@
 
 template <int N1, int KIND>
 static void launch_mode(H* h, const double* z, double* y, const MfmaTab* tab, const MfmaArgs& a, unsigned nb, int mode,
-                        double* dotp, const int* stop) {
+                        double* dotp, const int* stop, const double* w) {
   const double* fc = KIND == MFMA_WEIGHT || KIND == MFMA_TENSOR ? h->d_fw64 : h->d_fc64;
-  if (mode == 1)
-    hipLaunchKernelGGL((dg_mfma_kernel<N1, KIND, 1>), dim3(nb), dim3(256), 0, h->stream, z, y, fc, tab, a, nb, dotp, stop);
-  else if (mode == 2)
-    hipLaunchKernelGGL((dg_mfma_kernel<N1, KIND, 2>), dim3(nb), dim3(256), 0, h->stream, z, y, fc, tab, a, nb, dotp, stop);
-  else
-    hipLaunchKernelGGL((dg_mfma_kernel<N1, KIND, 0>), dim3(nb), dim3(256), 0, h->stream, z, y, fc, tab, a, nb, dotp, stop);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, h->stream, z, y, fc, tab, a, nb, dotp, stop, w);
+  };
+  switch (mode) {
+    case 1: run(dg_mfma_kernel<N1, KIND, 1>); break;
+    case 2: run(dg_mfma_kernel<N1, KIND, 2>); break;
+    case 3: run(dg_mfma_kernel<N1, KIND, 3>); break;
+    case 4: run(dg_mfma_kernel<N1, KIND, 4>); break;
+    case 5: run(dg_mfma_kernel<N1, KIND, 5>); break;
+    default: run(dg_mfma_kernel<N1, KIND, 0>); break;
+  }
 }
 
 template <int N1>
 static void launch_kind(H* h, const double* z, double* y, const MfmaTab* tab, const MfmaArgs& a, unsigned nb, int mode,
-                        double* dotp, const int* stop) {
+                        double* dotp, const int* stop, const double* w) {
   if (!h->vark) {
-    if (h->sym[0] && h->sym[1]) launch_mode<N1, MFMA_CONST>(h, z, y, tab, a, nb, mode, dotp, stop);
-    else launch_mode<N1, MFMA_CONV>(h, z, y, tab, a, nb, mode, dotp, stop);
+    if (h->sym[0] && h->sym[1]) launch_mode<N1, MFMA_CONST>(h, z, y, tab, a, nb, mode, dotp, stop, w);
+    else launch_mode<N1, MFMA_CONV>(h, z, y, tab, a, nb, mode, dotp, stop, w);
   }
-  else if (h->conv || !h->a64.weightsOn) launch_mode<N1, MFMA_GENERAL>(h, z, y, tab, a, nb, mode, dotp, stop);
-  else if (h->a64.aniso) launch_mode<N1, MFMA_TENSOR>(h, z, y, tab, a, nb, mode, dotp, stop);
-  else launch_mode<N1, MFMA_WEIGHT>(h, z, y, tab, a, nb, mode, dotp, stop);
+  else if (h->conv || !h->a64.weightsOn) launch_mode<N1, MFMA_GENERAL>(h, z, y, tab, a, nb, mode, dotp, stop, w);
+  else if (h->a64.aniso) launch_mode<N1, MFMA_TENSOR>(h, z, y, tab, a, nb, mode, dotp, stop, w);
+  else launch_mode<N1, MFMA_WEIGHT>(h, z, y, tab, a, nb, mode, dotp, stop, w);
 }
 
 // Arguments of one launch without the field's.
@@ -50,13 +55,14 @@ MfmaArgs mfma_args(const H* h, bool trans) {
   return a;
 }
 
-int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop) {
+int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop,
+                      const double* w) {
   const MfmaArgs a = mfma_args(h, trans);
   const unsigned nb = (unsigned)mfma_blocks(h);
   // J and J^T, each with the whole matrices and with their convection part (cell-wise kappa)
   const MfmaTab* tab = h->d_tab->mfma + (trans ? 1 : 0) + (h->vark ? 2 : 0);
-  if (h->n1 == 3) launch_kind<3>(h, z, y, tab, a, nb, mode, dotp, stop);
-  else launch_kind<4>(h, z, y, tab, a, nb, mode, dotp, stop);
+  if (h->n1 == 3) launch_kind<3>(h, z, y, tab, a, nb, mode, dotp, stop, w);
+  else launch_kind<4>(h, z, y, tab, a, nb, mode, dotp, stop, w);
   HIPCHK(h, hipGetLastError());
   return PDELAB_OK;
 }

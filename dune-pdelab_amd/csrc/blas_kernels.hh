@@ -36,15 +36,40 @@ __device__ __forceinline__ void block_sum(A (&v)[NR]) {
   }
 }
 
-// partial[b*NR + j] = block b's share of sum_i f_j(i)
-template <typename T, typename A>
+// Elements in flight per thread and stream of the reducing vector kernels: with one, the 1024
+// workgroups cannot cover the memory latency (x.y of 23.9M floats, 191 MB: 51 us, with four 29 us,
+// 6.5 TB/s).
+constexpr int kVecUnroll = 4;
+
+// partial[b] = block b's share of x.y, or partial[2 b + j] its shares of (x.y, y.y) (NR = 2)
+template <typename T, typename A, int NR>
 __global__ __launch_bounds__(kRedThreads) void dot_partial_kernel(const T* __restrict__ x, const T* __restrict__ y,
                                                                   long long n, A* __restrict__ partial) {
-  A v[1] = {A(0)};
-  for (long long i = (long long)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (long long)kRedBlocks * kRedThreads)
-    v[0] += (A)x[i] * (A)y[i];
-  block_sum<A, 1>(v);
-  if (threadIdx.x == 0) partial[blockIdx.x] = v[0];
+  A v[NR];
+#pragma unroll
+  for (int j = 0; j < NR; ++j) v[j] = A(0);
+  constexpr long long S = (long long)kRedBlocks * kRedThreads;
+  for (long long i0 = (long long)blockIdx.x * kRedThreads + threadIdx.x; i0 < n; i0 += kVecUnroll * S) {
+    T xv[kVecUnroll], yv[kVecUnroll];
+#pragma unroll
+    for (int u = 0; u < kVecUnroll; ++u) {
+      const long long i = i0 + u * S;
+      xv[u] = yv[u] = T(0);
+      if (i < n) {
+        xv[u] = x[i];
+        yv[u] = y[i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kVecUnroll; ++u) {
+      v[0] += (A)xv[u] * (A)yv[u];
+      if constexpr (NR == 2) v[1] += (A)yv[u] * (A)yv[u];
+    }
+  }
+  block_sum<A, NR>(v);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int j = 0; j < NR; ++j) partial[NR * blockIdx.x + j] = v[j];
 }
 
 // Single-workgroup sums of per-workgroup partials (up to tens of thousands of them):
@@ -169,7 +194,6 @@ __global__ __launch_bounds__(kRedThreads) void prec_dot_kernel(long long n, cons
 // scal[0] (cg_pq_kernel), cg_rupdate_kernel, cg_check_kernel and cg_xpupdate_kernel.
 // state = {stopped, aborted, stop iteration}; dstate = {defect, def0, reduction}. Every
 // kernel of an iteration after the one that stopped the loop returns at once.
-constexpr int kVecUnroll = 4;
 // Scalar slots of the step lengths: the single-workgroup kernels divide once, and the
 // vector kernels read the quotients (an FP64 division per wave cost ~10 us per launch).
 constexpr int kSlotLambda = 8, kSlotBeta = 9;
@@ -332,54 +356,21 @@ __global__ __launch_bounds__(256) void cg_pupdate_kernel(long long n, T* __restr
   }
 }
 
-// BiCGSTAB: p = r + beta (p - omega v)   (or p = r when first)
-template <typename T>
-__global__ __launch_bounds__(256) void bicg_p_kernel(long long n, T* __restrict__ p, const T* __restrict__ r,
-                                                     const T* __restrict__ v, T beta, T omega, int first) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    p[i] = first ? r[i] : beta * (p[i] - omega * v[i]) + r[i];
-}
-
-// x += a y; r -= a v; partials of r.r
-template <typename T, typename A>
-__global__ __launch_bounds__(kRedThreads) void xr_update_kernel(long long n, T* __restrict__ x, const T* __restrict__ y,
-                                                                T* __restrict__ r, const T* __restrict__ v, T a,
-                                                                A* __restrict__ partial) {
-  A s[1] = {A(0)};
-  for (long long i = (long long)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (long long)kRedBlocks * kRedThreads) {
-    x[i] += a * y[i];
-    const T ri = r[i] - a * v[i];
-    r[i] = ri;
-    s[0] += (A)ri * (A)ri;
-  }
-  block_sum<A, 1>(s);
-  if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
-}
-
-// partials of t.r and t.t
-template <typename T, typename A>
-__global__ __launch_bounds__(kRedThreads) void dot2_kernel(long long n, const T* __restrict__ t, const T* __restrict__ r,
-                                                           A* __restrict__ partial) {
-  A s[2] = {A(0), A(0)};
-  for (long long i = (long long)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (long long)kRedBlocks * kRedThreads) {
-    const A ti = (A)t[i];
-    s[0] += ti * (A)r[i];
-    s[1] += ti * ti;
-  }
-  block_sum<A, 2>(s);
-  if (threadIdx.x == 0) { partial[2 * blockIdx.x] = s[0]; partial[2 * blockIdx.x + 1] = s[1]; }
-}
-
 // ---------------------------------------------------------------------------
 // Device-side BiCGSTAB (dune-istl BiCGSTABSolver::apply with its half-step Iteration
-// counting). Per iteration: p update, W^{-1} p, the apply, rt.v, x/r update with the r.r
-// partials, the half-step check, W^{-1} r, the apply, (t.r, t.t), x/r update with the
-// (r.r, rt.r) partials and the full-step check; single-workgroup kernels keep the solver's
-// scalars in FP64 as the host loop kept them:
+// counting). Per iteration: y1 = W^{-1} p, v = J y1 with rt.v, r -= alpha v with r.r, the
+// half-step check, y2 = W^{-1} r, t = J y2 with (r.t, t.t), x += alpha y1 + omega y2 and
+// r -= omega t with (r.r, rt.r), the full-step check. The loop is bound by these streams, so
+// point Jacobi works inside the updates, p is kept only for a preconditioner with a launch of
+// its own, x is updated once and the FP64 matrix-core apply takes the dots: 24 vectors read or
+// written per iteration where one kernel per statement moved 31 (96^3 Q2 convection, 191 MB per
+// vector: 1130 -> 920 us per iteration; the updates run at 5.8 to 6.3 TB/s). Single-workgroup
+// kernels keep the solver's scalars in FP64:
 //   bs = {rho, rho_new, alpha, omega, beta}; state = {stopped, abort code, half steps};
 //   dstate = {defect, def0, reduction}.
-// Once state[0] is set every later kernel that writes x, r or the scalars returns at once,
-// so x and r are those of the half step at which the loop stopped.
+// Once state[0] is set every later kernel that writes x, r or the scalars returns at once, but
+// for the alpha part of x when it was the half step that stopped the loop: x and r are those of
+// the half step at which it stopped.
 enum { BICG_RUNNING = 0, BICG_NAN = 1, BICG_RHO = 2, BICG_OMEGA = 3, BICG_H = 4 };
 constexpr int kBsRho = 0, kBsRhoNew = 1, kBsAlpha = 2, kBsOmega = 3, kBsBeta = 4;
 constexpr double kBicgEps = 1e-80;  // dune-istl's EPSILON of BiCGSTABSolver
@@ -411,15 +402,40 @@ __global__ __launch_bounds__(64) void bicg_init_kernel(double* __restrict__ bs, 
   }
 }
 
-// p = r (first iteration) or p = r + beta (p - omega v)
-template <typename T>
-__global__ __launch_bounds__(256) void bicg_p_dev_kernel(long long n, T* __restrict__ p, const T* __restrict__ r,
-                                                         const T* __restrict__ v, const double* __restrict__ bs,
-                                                         const int* __restrict__ state, int first) {
+// p = r (first iteration) or p = r + beta (p - omega v); with POINT the preconditioned
+// direction y = dinv p in p's place: y = dinv r or y = dinv (r - beta omega v) + beta y. One
+// element per thread over an exact grid, as in cg_xpupdate_kernel.
+template <typename T, bool POINT>
+__global__ __launch_bounds__(256) void bicg_dir_kernel(long long n, T* __restrict__ p, const T* __restrict__ r,
+                                                       const T* __restrict__ v, const T* __restrict__ dinv,
+                                                       const double* __restrict__ bs, const int* __restrict__ state,
+                                                       int first) {
+  constexpr int E = xp_ept<T>();
+  typedef T V __attribute__((ext_vector_type(E)));
   if (state[0]) return;
-  const T beta = (T)bs[kBsBeta], omega = (T)bs[kBsOmega];
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    p[i] = first ? r[i] : beta * (p[i] - omega * v[i]) + r[i];
+  const T beta = (T)bs[kBsBeta], omega = (T)bs[kBsOmega], bo = beta * omega;
+  const long long i0 = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * E;
+  if (i0 >= n) return;
+  if (i0 + E <= n) {
+    V pn = *reinterpret_cast<const V*>(r + i0);
+    V d;
+    if constexpr (POINT) d = *reinterpret_cast<const V*>(dinv + i0);
+    if (!first) {
+      const V po = *reinterpret_cast<const V*>(p + i0), vo = ld_stream<V>(reinterpret_cast<const V*>(v + i0));
+      if constexpr (POINT) pn = d * (pn - bo * vo) + beta * po;
+      else pn = beta * (po - omega * vo) + pn;
+    } else if constexpr (POINT) pn = d * pn;
+    *reinterpret_cast<V*>(p + i0) = pn;
+    return;
+  }
+  for (long long i = i0; i < n; ++i) {  // an odd last float
+    T pn = r[i];
+    if (!first) {
+      if constexpr (POINT) pn = dinv[i] * (pn - bo * v[i]) + beta * p[i];
+      else pn = beta * (p[i] - omega * v[i]) + pn;
+    } else if constexpr (POINT) pn = dinv[i] * pn;
+    p[i] = pn;
+  }
 }
 
 // y = dinv .* x (or y = x), skipped once the loop has stopped
@@ -431,36 +447,101 @@ __global__ __launch_bounds__(256) void prec_stop_kernel(long long n, const T* __
     y[i] = dinv ? dinv[i] * x[i] : x[i];
 }
 
-// x += a y; r -= a v with a = bs[slot]; partials of r.r (NR = 1) or of (r.r, rt.r) (NR = 2),
-// in the order of xr_update_kernel and dot_partial_kernel
-template <typename T, typename A, int NR>
-__global__ __launch_bounds__(kRedThreads) void bicg_xr_kernel(long long n, T* __restrict__ x, const T* __restrict__ y,
-                                                              T* __restrict__ r, const T* __restrict__ v,
-                                                              const T* __restrict__ rt, const double* __restrict__ bs,
-                                                              int slot, A* __restrict__ partial,
-                                                              const int* __restrict__ state) {
+// First half step: r -= alpha v with the r.r partials; with POINT also y = dinv r
+template <typename T, typename A, bool POINT>
+__global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* __restrict__ r, const T* __restrict__ v,
+                                                                const T* __restrict__ dinv, T* __restrict__ y,
+                                                                const double* __restrict__ bs, A* __restrict__ partial,
+                                                                const int* __restrict__ state) {
   if (state[0]) return;
-  const T a = (T)bs[slot];
-  A s[NR];
+  const T alpha = (T)bs[kBsAlpha];
+  A s[1] = {A(0)};
+  constexpr long long S = (long long)kRedBlocks * kRedThreads;
+  for (long long i0 = (long long)blockIdx.x * kRedThreads + threadIdx.x; i0 < n; i0 += kVecUnroll * S) {
+    T rv[kVecUnroll], vv[kVecUnroll], dv[kVecUnroll];
 #pragma unroll
-  for (int j = 0; j < NR; ++j) s[j] = A(0);
-  for (long long i = (long long)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (long long)kRedBlocks * kRedThreads) {
-    x[i] += a * y[i];
-    const T ri = r[i] - a * v[i];
-    r[i] = ri;
-    s[0] += (A)ri * (A)ri;
-    if constexpr (NR == 2) s[1] += (A)rt[i] * (A)ri;
+    for (int u = 0; u < kVecUnroll; ++u) {
+      const long long i = i0 + u * S;
+      rv[u] = vv[u] = dv[u] = T(0);
+      if (i < n) {
+        rv[u] = r[i];
+        vv[u] = v[i];
+        if constexpr (POINT) dv[u] = dinv[i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kVecUnroll; ++u) {
+      const long long i = i0 + u * S;
+      if (i < n) {
+        const T ri = rv[u] - alpha * vv[u];
+        r[i] = ri;
+        if constexpr (POINT) y[i] = dv[u] * ri;
+        s[0] += (A)ri * (A)ri;
+      }
+    }
   }
-  block_sum<A, NR>(s);
-  if (threadIdx.x == 0)
+  block_sum<A, 1>(s);
+  if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
+}
+
+// Second half step `half`: x += alpha y1 + omega y2, r -= omega t with the (r.r, rt.r)
+// partials; y2 null: r before its update (no preconditioner); y1 null: its part is in x already.
+// If the first half step stopped the loop, only x += alpha y1.
+template <typename T, typename A>
+__global__ __launch_bounds__(kRedThreads) void bicg_full_kernel(long long n, T* __restrict__ x, const T* __restrict__ y1,
+                                                                const T* __restrict__ y2, T* __restrict__ r,
+                                                                const T* __restrict__ t, const T* __restrict__ rt,
+                                                                const double* __restrict__ bs, A* __restrict__ partial,
+                                                                const int* __restrict__ state, int half) {
+  const long long first = (long long)blockIdx.x * kRedThreads + threadIdx.x;
+  constexpr long long S = (long long)kRedBlocks * kRedThreads;
+  const T alpha = (T)bs[kBsAlpha], omega = (T)bs[kBsOmega];
+  if (state[0]) {
+    if (state[2] == half - 1 && y1)
+      for (long long i = first; i < n; i += S) x[i] += alpha * y1[i];
+    return;
+  }
+  A s[2] = {A(0), A(0)};
+  for (long long i0 = first; i0 < n; i0 += kVecUnroll * S) {
+    T xv[kVecUnroll], av[kVecUnroll], bv[kVecUnroll], rv[kVecUnroll], tv[kVecUnroll], sv[kVecUnroll];
 #pragma unroll
-    for (int j = 0; j < NR; ++j) partial[NR * blockIdx.x + j] = s[j];
+    for (int u = 0; u < kVecUnroll; ++u) {
+      const long long i = i0 + u * S;
+      xv[u] = av[u] = bv[u] = rv[u] = tv[u] = sv[u] = T(0);
+      if (i < n) {
+        xv[u] = ld_stream<T>(x + i);
+        if (y1) av[u] = y1[i];
+        rv[u] = r[i];
+        bv[u] = y2 ? ld_stream<T>(y2 + i) : rv[u];
+        tv[u] = ld_stream<T>(t + i);
+        sv[u] = ld_stream<T>(rt + i);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kVecUnroll; ++u) {
+      const long long i = i0 + u * S;
+      if (i < n) {
+        T xi = xv[u];
+        if (y1) xi += alpha * av[u];
+        st_stream<T>(xi + omega * bv[u], x + i);
+        const T ri = rv[u] - omega * tv[u];
+        r[i] = ri;
+        s[0] += (A)ri * (A)ri;
+        s[1] += (A)sv[u] * (A)ri;
+      }
+    }
+  }
+  block_sum<A, 2>(s);
+  if (threadIdx.x == 0) {
+    partial[2 * blockIdx.x] = s[0];
+    partial[2 * blockIdx.x + 1] = s[1];
+  }
 }
 
 // The scalar steps, one workgroup reducing the partials first:
 //   PHASE 0: h = rt.v; |h| < EPSILON aborts; alpha = rho_new / h (0 when the defect is 0)
 //   PHASE 1: defect of the half step, Iteration::step
-//   PHASE 2: omega = t.r / t.t (0 when the defect is 0)
+//   PHASE 2: omega = r.t / t.t (0 when the defect is 0)
 //   PHASE 3: defect of the full step, rho = rho_new, rho_new = rt.r, Iteration::step; then
 //            the breakdown checks at the top of dune-istl's next iteration (|rho|, |omega|
 //            <= EPSILON) and beta = (rho_new / rho)(alpha / omega)

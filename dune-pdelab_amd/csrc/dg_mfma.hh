@@ -104,10 +104,11 @@ constexpr int mfma_row(bool tensor) { return tensor ? 6 : 4; }  // values of a c
 // Waves per SIMD the register allocation aims at: no instance spills. (With 96 bytes of scratch
 // the face-weight Q3 kernel took 97 instead of 76 us at 64^3, and 72 bytes cost the fused-dot
 // Q2 one 5 of 17 us at 32^3.)
-template <int N1, int KIND>
+template <int N1, int KIND, int MODE>
 constexpr int mfma_waves() {
   if (KIND == MFMA_GENERAL) return 2;
   if (KIND == MFMA_TENSOR) return N1 == 4 ? 2 : 3;
+  if (KIND == MFMA_WEIGHT && N1 == 4) return MODE < 3 ? 3 : 2;
   return KIND == MFMA_WEIGHT || N1 == 4 ? 3 : 4;
 }
 
@@ -207,6 +208,10 @@ struct MfmaStage {
     if constexpr (N1 == 4) return *reinterpret_cast<const mfma_a2*>(buf + a);
     else return buf[a];
   }
+  __device__ static __forceinline__ double dot(const E& u, const E& v) {
+    if constexpr (N1 == 4) return u.x * v.x + u.y * v.y;
+    else return u * v;
+  }
   __device__ static __forceinline__ E load(mfma_gp base, unsigned off) {
     typedef const E __attribute__((address_space(1))) * EP;
     return *(EP)((const char __attribute__((address_space(1)))*)base + here(off));
@@ -243,7 +248,11 @@ __device__ __forceinline__ double dpp_upper_pair(double src) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// MODE 0: y = J z, 1: y += J z, 2: y = J z and partials of z . (J z), one per workgroup.
+// MODE 0: y = J z, 1: y += J z, 2: y = J z and partials of z . (J z), one per workgroup. With a
+// second vector w (wvec), read as y is in mode 1:
+// 3: y = J z and partials of w . y, 4: y = J z and partials of (w . y, y . y), 5: y += J z + w.
+// (A pass of its own reads y back. 96^3 Q2: a dot 74 us, here 35 more; 64^3 Q3 lognormal residual:
+// apply and axpy 154 us, mode 5 110 us, 4.9 TB/s.)
 // VEL 1 (J), 2 (J^T): adds the convection terms of the velocity field at M points per direction
 // (dg_velocity.hh states them). They too are 4x4x4 products: z at the points by contracting x
 // in registers, z (T0 -> T1) and y; the products with b; and the tests back, y (T1 -> T0) and z.
@@ -251,10 +260,11 @@ __device__ __forceinline__ double dpp_upper_pair(double src) {
 // neighbour's / upper neighbour's along lane%4 (T1 -> lane/16 = z), interpolated, upwinded with a
 // quad permutation and tested back; the z faces likewise from T0, the x faces per register.
 template <int N1, int KIND, int MODE, int VEL = 0, int M = N1>
-__global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mfma_kernel(const double* __restrict__ z, double* __restrict__ y,
+__global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND, MODE>())) void dg_mfma_kernel(const double* __restrict__ z, double* __restrict__ y,
                                                       const double* __restrict__ fc, const MfmaTab* __restrict__ tab,
                                                       const MfmaArgs a, unsigned nblocks, double* __restrict__ dotp,
-                                                      const int* __restrict__ stop) {
+                                                      const int* __restrict__ stop,
+                                                      const double* __restrict__ wvec = nullptr) {
   // a device-side Krylov loop that has stopped: read here, obeyed once the first loads are on
   // their way (the flag and they come from beyond the L2, which other XCDs' kernels have written)
   const int stopped = stop ? *stop : 0;
@@ -263,6 +273,7 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mf
   constexpr int NL = SG::NL;
   constexpr unsigned CB = NL * sizeof(double);
   constexpr bool WT = KIND == MFMA_WEIGHT || KIND == MFMA_TENSOR;  // face weights
+  constexpr bool RY = MODE == 1 || MODE == 5, RW = MODE >= 3;      // y or w is read
   constexpr bool ADD = !WT;                                        // the tables' line matrices take part
   constexpr int FW = mfma_row(KIND == MFMA_TENSOR), FK = FW - 3;
   __shared__ __attribute__((aligned(16))) double lds[4 * SG::WAVE];
@@ -372,9 +383,9 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mf
     return a.S[2] * (f[0] * tab->X[0][me] + f[2] * tab->X[1][me] + f[1] * tab->X[2][me]) + Nzl;
   };
   // in flight for the next step: elements of the next plane, the y-neighbours and the end cells,
-  // of y (MODE 1), and the face weights. They are issued in one batch and waited for together:
+  // of y and w, and the face weights. They are issued in one batch and waited for together:
   // loads complete in order, so a load issued later would have to wait for these.
-  E rn[2], rl[2], rr[2], rx, ry[2];
+  E rn[2], rl[2], rr[2], rx, ry[2], rw[2];
   double fk[3] = {0, 0, 0}, fx = 0, fy = 0, fxu = 0, fyu = 0, fzu = 0;
   auto fetch = [&](const double* base, const unsigned (&o)[2], E (&v)[2]) {
     const mfma_gp b = per_step<mfma_gp>(base);
@@ -387,7 +398,8 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mf
     fetch(zk, oyl, rl);
     fetch(zk, oyr, rr);
     if (ldx) rx = SG::load(per_step<mfma_gp>(zk), ox);
-    if constexpr (MODE == 1) fetch(y + (size_t)kz * plane, ow, ry);
+    if constexpr (RY) fetch(y + (size_t)kz * plane, ow, ry);
+    if constexpr (RW) fetch(wvec + (size_t)kz * plane, ow, rw);
     if constexpr (WT) {
       const mfma_gp f = per_step<mfma_gp>(fc + (size_t)kz * a.np * FW);
       const unsigned of = cc * (unsigned)(FW * 8);
@@ -621,7 +633,7 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mf
     const bool keep = i * N1 + j <= (N1 - 1 - i) * N1 + (N1 - 1 - j);
     return m[keep ? i : N1 - 1 - i][keep ? j : N1 - 1 - j];
   };
-  double pq = 0;
+  double pq = 0, qq = 0;  // this lane's shares of the dots
   // one z-step: own cells in B0 (T0 lines uz), the next plane's to B1 (T0 lines zr)
   auto step = [&](int kz, double* B0, double* B1, double (&uz)[N1], double (&zr)[N1]) {
     const bool loz = kz > 0, hiz = kz < a.nz - 1;
@@ -632,10 +644,17 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mf
     put(BYR, rr);
     if (ldx) SG::put(BX, sx, rx);
     const double kx = fk[0], ky = fk[1], kz_ = fk[2], wxl = fx, wyl = fy, wxu = hix ? fxu : 0.0, wyu = hiy ? fyu : 0.0, wzu = hiz ? fzu : 0.0;
-    E yo[2];
-    if constexpr (MODE == 1) {
+    E yo[2], wo[2];
+    if constexpr (RY) {
       yo[0] = ry[0];
       yo[1] = ry[1];
+    }
+    if constexpr (MODE == 5) {
+      yo[0] += rw[0];
+      if (two) yo[1] += rw[1];
+    } else if constexpr (RW) {
+      wo[0] = rw[0];
+      wo[1] = rw[1];
     }
     if (kz + 1 < k1) fetch_step(kz + 1);
     wave_lds_fence();
@@ -861,7 +880,9 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mf
       for (int p = 0; p < 2; ++p) {
         if ((p == 0 || two) && st[p]) {
           E v = SG::get(BYL, se[p]);
-          if constexpr (MODE == 1) v += yo[p];
+          if constexpr (MODE == 3 || MODE == 4) pq += SG::dot(wo[p], v);
+          if constexpr (MODE == 4) qq += SG::dot(v, v);
+          if constexpr (RY) v += yo[p];
           SG::store(yc, ow[p], v);
         }
       }
@@ -874,10 +895,18 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND>())) void dg_mf
     step(kz + 1, W1, W, ub, ua);
   }
   if (kz < k1) step(kz, W, W1, ua, ub);
-  if constexpr (MODE == 2) {
+  if constexpr (MODE == 2 || MODE == 3) {
     double v[1] = {pq};
     block_sum_reuse<4, double, 1>(v, lds);
     if (threadIdx.x == 0) dotp[blockIdx.x] = v[0];
+  }
+  if constexpr (MODE == 4) {
+    double v[2] = {pq, qq};
+    block_sum_reuse<4, double, 2>(v, lds);
+    if (threadIdx.x == 0) {
+      dotp[2 * blockIdx.x] = v[0];
+      dotp[2 * blockIdx.x + 1] = v[1];
+    }
   }
 }
 

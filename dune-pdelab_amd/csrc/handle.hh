@@ -263,9 +263,11 @@ template <int N1, typename T>
 int launch_apply_n(H* h, const T* z, T* y, const T* fc, const DGArgs<T>& a, bool trans, int mode, T* dotp,
                    const int* stop);
 
-// The FP64 apply on the matrix cores (apply_mfma.hip; modes as above) and its constants, from
-// the 1D matrices of J and J^T without reaction and their convection parts.
-int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop);
+// The FP64 apply on the matrix cores (apply_mfma.hip; modes as above and, with a vector w,
+// 3: w.y partials, 4: (w.y, y.y) partials, 5: y += J z + w) and its constants, from the 1D
+// matrices of J and J^T without reaction and their convection parts.
+int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, double* dotp, const int* stop,
+                      const double* w = nullptr);
 void mfma_setup(H* h, const DGArgs<long double>& al, const LineMats<long double> (&m)[2],
                 const LineMats<long double> (&mconv)[2], MfmaTab (&t)[4]);
 MfmaArgs mfma_args(const H* h, bool trans);

@@ -490,7 +490,7 @@ static int read_scalars(H* h, A* out, int count) {
 
 template <typename T, typename A>
 static int dot_dev(H* h, const T* x, const T* y, long long n, int slot) {
-  hipLaunchKernelGGL((dot_partial_kernel<T, A>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, x, y, n,
+  hipLaunchKernelGGL((dot_partial_kernel<T, A, 1>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, x, y, n,
                      partial_buf<A>(h));
   HIPCHK(h, hipGetLastError());
   return finish_reduce<A, 1>(h, slot);
@@ -552,6 +552,7 @@ struct Prec {
   bool block() const { return kind == PDELAB_PREC_BLOCK_JACOBI; }
   bool sor() const { return kind == PDELAB_PREC_BLOCK_SOR; }
   bool ibj() const { return kind == PDELAB_PREC_ITERATIVE_BLOCK_JACOBI; }
+  bool launched() const { return block() || sor() || ibj(); }  // by launches of its own
 };
 
 // The cached point diagonal and block Jacobi data belong to the operator with the current
@@ -602,6 +603,15 @@ static int prec_dot(H* h, const Prec<T>& P, const T* in, T* out, int slot) {
   return PDELAB_OK;
 }
 
+// The partials of the apply's dots, sized for every kernel (the choice can change with
+// set_kappa and with the precision) and for two sums.
+static int ensure_applydot(H* h) {
+  if (h->d_applydot) return PDELAB_OK;
+  const long long nmax = std::max({apply_blocks_of(h, true), apply_blocks_of(h, false), 2 * mfma_blocks(h), 1LL});
+  HIPCHK(h, hipMalloc(&h->d_applydot, sizeof(double) * (size_t)nmax));
+  return PDELAB_OK;
+}
+
 // Iterations between host reads of the device CG loop's stop flag.
 constexpr int kCheckEvery = 16;
 
@@ -622,11 +632,7 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
                    double red, CgLoopOut& out) {
   const long long n = h->N;
   const long long nbapply = apply_partials<T>(h);
-  // sized for every kernel: the choice can change with set_kappa and with the precision
-  if (!h->d_applydot) {
-    const long long nmax = std::max({apply_blocks_of(h, true), apply_blocks_of(h, false), mfma_blocks(h), 1LL});
-    HIPCHK(h, hipMalloc(&h->d_applydot, sizeof(double) * (size_t)nmax));
-  }
+  CHK(ensure_applydot(h));
   static_assert(std::is_same<T, A>::value, "the fused apply dot is accumulated in the vector type");
   A* scal = scal_buf<A>(h);
   T* dotp = reinterpret_cast<T*>(h->d_applydot);
@@ -739,27 +745,139 @@ static int cg_solve(H* h, T* x, T* b, double reduction, int maxit, int precond, 
 // Iterations of the device BiCGSTAB loop between host reads of its stop flag.
 constexpr int kBicgCheckEvery = 8;
 
+// Vectors of a BiCGSTAB run (blas_kernels.hh). A point preconditioner keeps y1 in p's place;
+// without a preconditioner y2 is r.
+template <typename T>
+struct BicgVecs {
+  T *x, *r, *p, *v, *t, *y1, *y2, *rt;
+};
+
+// p, v, t, y2, rt of the workspace slots base .. base+4 and, for a preconditioner with a launch
+// of its own, y1 of slot 7.
+template <typename T>
+static int bicg_vecs(H* h, const Prec<T>& P, int base, T* x, T* r, BicgVecs<T>& w) {
+  CHK(ensure_ws<T>(h, base + 5));
+  T** s = ws<T>(h);
+  w = {x, r, s[base], s[base + 1], s[base + 2], s[base], s[base + 3], s[base + 4]};
+  if (P.launched()) {
+    if (!s[7]) HIPCHK(h, hipMalloc(&s[7], sizeof(T) * h->N));
+    w.y1 = s[7];
+  } else if (!P.dinv) w.y2 = r;
+  if (!h->d_bscal) HIPCHK(h, hipMalloc(&h->d_bscal, sizeof(double) * 8));
+  return ensure_applydot(h);
+}
+
+// out = W^{-1} in of a BiCGSTAB loop, skipped once it has stopped (y2 = r needs no launch)
+template <typename T, typename A>
+static int bicg_prec(H* h, const Prec<T>& P, const T* in, T* out) {
+  int* st = h->d_state;
+  if (P.sor()) return sor_launch<T>(h, in, out, st, false);
+  if (P.ibj()) return ibj_launch<T>(h, in, out, static_cast<int*>(h->d_ibj_stat), nullptr, st, false);
+  if (P.block()) {
+    const BJVec<T, A> bv{in, out, nullptr, nullptr, nullptr, nullptr, st};
+    return bj_launch<T, A>(h, P.trans, BJ_PREC, bv, nullptr);
+  }
+  if (P.dinv)
+    hipLaunchKernelGGL(prec_stop_kernel<T>, dim3(grid_for(h->N)), dim3(256), 0, h->stream, h->N, P.dinv, in, out,
+                       (const int*)st);
+  HIPCHK(h, hipGetLastError());
+  return PDELAB_OK;
+}
+
+// y = J z (or J^T z) and the partials of w.y (NR = 1) or (w.y, y.y): inside the apply on the
+// matrix cores, else by a pass of its own.
+template <typename T, typename A, int NR>
+static int apply_dots(H* h, const T* z, T* y, bool trans, const T* w, const A** parts, int* nparts) {
+  if constexpr (std::is_same<T, double>::value) {
+    if (!h->varb && mfma_kernel(h)) {
+      CHK(check_outflow(h));
+      *parts = h->d_applydot;
+      *nparts = (int)mfma_blocks(h);
+      return launch_apply_mfma(h, z, y, trans, NR == 1 ? 3 : 4, h->d_applydot, h->d_state, w);
+    }
+  }
+  CHK(apply_mode<T>(h, z, y, trans, 0, nullptr, h->d_state));
+  hipLaunchKernelGGL((dot_partial_kernel<T, A, NR>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, w, (const T*)y,
+                     h->N, partial_buf<A>(h));
+  HIPCHK(h, hipGetLastError());
+  *parts = partial_buf<A>(h);
+  *nparts = kRedBlocks;
+  return PDELAB_OK;
+}
+
+template <typename A, int PHASE>
+static void bicg_scalar(H* h, const A* parts, int nparts, int half) {
+  hipLaunchKernelGGL((bicg_scalar_kernel<A, PHASE>), dim3(1), dim3(kFinalThreads), 0, h->stream, parts, nparts,
+                     h->d_bscal, h->d_state, h->d_dstate, half);
+}
+
+// First half step of iteration i: p, y1 = W^{-1} p, v = J y1, alpha, r -= alpha v
+template <typename T, typename A>
+static int bicg_first_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool first, int i) {
+  const long long n = h->N;
+  const dim3 grid((unsigned)((n + 256LL * xp_ept<T>() - 1) / (256LL * xp_ept<T>())));
+  const double* bs = h->d_bscal;
+  const int* st = h->d_state;
+  const T *r = w.r, *v = w.v;
+  const bool point = P.dinv != nullptr;
+  if (point)
+    hipLaunchKernelGGL((bicg_dir_kernel<T, true>), grid, dim3(256), 0, h->stream, n, w.p, r, v, P.dinv, bs, st, first);
+  else
+    hipLaunchKernelGGL((bicg_dir_kernel<T, false>), grid, dim3(256), 0, h->stream, n, w.p, r, v, P.dinv, bs, st, first);
+  if (P.launched()) CHK((bicg_prec<T, A>(h, P, w.p, w.y1)));
+  const A* parts;
+  int np;
+  CHK((apply_dots<T, A, 1>(h, w.y1, w.v, P.trans, w.rt, &parts, &np)));
+  bicg_scalar<A, 0>(h, parts, np, 2 * i - 1);
+  A* part = partial_buf<A>(h);
+  if (point)
+    hipLaunchKernelGGL((bicg_half_kernel<T, A, true>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, w.r, v, P.dinv,
+                       w.y2, bs, part, st);
+  else
+    hipLaunchKernelGGL((bicg_half_kernel<T, A, false>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, w.r, v,
+                       P.dinv, (T*)nullptr, bs, part, st);
+  bicg_scalar<A, 1>(h, part, kRedBlocks, 2 * i - 1);
+  HIPCHK(h, hipGetLastError());
+  return PDELAB_OK;
+}
+
+// Second half step of iteration i: y2 = W^{-1} r, t = J y2, omega, x += alpha y1 + omega y2,
+// r -= omega t, rho. resumed: r is new since the first half step and x has its part.
+template <typename T, typename A>
+static int bicg_second_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool resumed, int i) {
+  if (P.launched() || resumed) CHK((bicg_prec<T, A>(h, P, w.r, w.y2)));
+  const A* parts;
+  int np;
+  CHK((apply_dots<T, A, 2>(h, w.y2, w.t, P.trans, w.r, &parts, &np)));
+  bicg_scalar<A, 2>(h, parts, np, 2 * i);
+  A* part = partial_buf<A>(h);
+  hipLaunchKernelGGL((bicg_full_kernel<T, A>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, h->N, w.x,
+                     resumed ? (const T*)nullptr : (const T*)w.y1, w.y2 == w.r ? (const T*)nullptr : (const T*)w.y2, w.r,
+                     (const T*)w.t, (const T*)w.rt, (const double*)h->d_bscal, part, (const int*)h->d_state, 2 * i);
+  bicg_scalar<A, 3>(h, part, kRedBlocks, 2 * i);
+  HIPCHK(h, hipGetLastError());
+  return PDELAB_OK;
+}
+
 // BiCGSTABSolver::apply (dune-istl) with half-step iteration counting, as a device-side
 // loop: the scalars, the Iteration::step test and the breakdown checks run in
-// single-workgroup kernels (bicg_scalar_kernel), so an iteration enqueues its 13 launches
-// without waiting; the host reads the stop flag every kBicgCheckEvery iterations.
-// Workspace slots base .. base+4 (p, v, t, y, rt).
+// single-workgroup kernels (bicg_scalar_kernel), so an iteration enqueues its launches (9 on the
+// matrix-core path with point Jacobi) without waiting; the host reads the stop flag every
+// kBicgCheckEvery iterations.
 template <typename T, typename A>
 static int bicgstab_solve(H* h, T* x, T* r, double reduction, int maxit, int precond, bool trans, int base,
                           pdelab_linear_solver_result* res) {
   auto t0 = std::chrono::steady_clock::now();
   const long long n = h->N;
-  CHK(ensure_ws<T>(h, base + 5));
-  T *p = ws<T>(h)[base], *v = ws<T>(h)[base + 1], *t = ws<T>(h)[base + 2], *y = ws<T>(h)[base + 3],
-    *rt = ws<T>(h)[base + 4];
   Prec<T> P;
   CHK(make_prec<T>(h, precond, trans, P));
-  if (!h->d_bscal) HIPCHK(h, hipMalloc(&h->d_bscal, sizeof(double) * 8));
+  BicgVecs<T> w;
+  CHK(bicg_vecs<T>(h, P, base, x, r, w));
   Iter iter(reduction);
   int status = PDELAB_OK;
-  CHK(apply_t<T>(h, x, t, trans, false));
-  hipLaunchKernelGGL(axpy_kernel<T>, dim3(grid_for(n)), dim3(256), 0, h->stream, n, T(-1), (const T*)t, r);
-  HIPCHK(h, hipMemcpyAsync(rt, r, sizeof(T) * n, hipMemcpyDeviceToDevice, h->stream));
+  CHK(apply_t<T>(h, x, w.t, trans, false));
+  hipLaunchKernelGGL(axpy_kernel<T>, dim3(grid_for(n)), dim3(256), 0, h->stream, n, T(-1), (const T*)w.t, r);
+  HIPCHK(h, hipMemcpyAsync(w.rt, r, sizeof(T) * n, hipMemcpyDeviceToDevice, h->stream));
   CHK(dot_dev<T, A>(h, r, r, n, 0));
   A sc[4];
   CHK(read_scalars<A>(h, sc, 1));
@@ -777,46 +895,11 @@ static int bicgstab_solve(H* h, T* x, T* r, double reduction, int maxit, int pre
     h->h_dstate[3] = 0.0;
     HIPCHK(h, hipMemcpyAsync(st, h->h_state, sizeof(int) * 4, hipMemcpyHostToDevice, h->stream));
     HIPCHK(h, hipMemcpyAsync(ds, h->h_dstate, sizeof(double) * 4, hipMemcpyHostToDevice, h->stream));
-    A* part = partial_buf<A>(h);
-    const dim3 rg(kRedBlocks), rb(kRedThreads), fg(1), fb(kFinalThreads);
     if (P.ibj()) HIPCHK(h, hipMemsetAsync(h->d_ibj_stat, 0, 16, h->stream));
-    auto prec = [&](const T* in, T* out) -> int {
-      if (P.sor()) return sor_launch<T>(h, in, out, st, false);
-      if (P.ibj()) return ibj_launch<T>(h, in, out, static_cast<int*>(h->d_ibj_stat), nullptr, st, false);
-      if (P.block()) {
-        const BJVec<T, A> bv{in, out, nullptr, nullptr, nullptr, nullptr, st};
-        return bj_launch<T, A>(h, P.trans, BJ_PREC, bv, nullptr);
-      }
-      hipLaunchKernelGGL(prec_stop_kernel<T>, dim3(grid_for(n)), dim3(256), 0, h->stream, n, P.dinv, in, out,
-                         (const int*)st);
-      HIPCHK(h, hipGetLastError());
-      return PDELAB_OK;
-    };
     bool stopped = false;
     for (int i = 1; i <= maxit && !stopped; ++i) {
-      // first half step: p, y = W^{-1} p, v = J y, alpha, x += alpha y, r -= alpha v
-      hipLaunchKernelGGL(bicg_p_dev_kernel<T>, dim3(grid_for(n)), dim3(256), 0, h->stream, n, p, (const T*)r,
-                         (const T*)v, (const double*)bs, (const int*)st, i == 1 ? 1 : 0);
-      CHK(prec(p, y));
-      CHK(apply_mode<T>(h, y, v, trans, 0, nullptr, st));
-      hipLaunchKernelGGL((dot_partial_kernel<T, A>), rg, rb, 0, h->stream, (const T*)rt, (const T*)v, n, part);
-      hipLaunchKernelGGL((bicg_scalar_kernel<A, 0>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                         2 * i - 1);
-      hipLaunchKernelGGL((bicg_xr_kernel<T, A, 1>), rg, rb, 0, h->stream, n, x, (const T*)y, r, (const T*)v,
-                         (const T*)nullptr, (const double*)bs, kBsAlpha, part, (const int*)st);
-      hipLaunchKernelGGL((bicg_scalar_kernel<A, 1>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                         2 * i - 1);
-      // second half step: y = W^{-1} r, t = J y, omega, x += omega y, r -= omega t, rho
-      CHK(prec(r, y));
-      CHK(apply_mode<T>(h, y, t, trans, 0, nullptr, st));
-      hipLaunchKernelGGL((dot2_kernel<T, A>), rg, rb, 0, h->stream, n, (const T*)t, (const T*)r, part);
-      hipLaunchKernelGGL((bicg_scalar_kernel<A, 2>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                         2 * i);
-      hipLaunchKernelGGL((bicg_xr_kernel<T, A, 2>), rg, rb, 0, h->stream, n, x, (const T*)y, r, (const T*)t,
-                         (const T*)rt, (const double*)bs, kBsOmega, part, (const int*)st);
-      hipLaunchKernelGGL((bicg_scalar_kernel<A, 3>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                         2 * i);
-      HIPCHK(h, hipGetLastError());
+      CHK((bicg_first_half<T, A>(h, P, w, i == 1, i)));
+      CHK((bicg_second_half<T, A>(h, P, w, false, i)));
       if (i % kBicgCheckEvery == 0 || i == maxit) {
         HIPCHK(h, hipMemcpyAsync(h->h_state, st, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -1149,16 +1232,14 @@ static int bicgstab_mixed_reliable(H* h, int precond, double inner_reduction, in
   Prec<T> P;
   CHK(make_prec<T>(h, precond, false, P));
   CHK(ensure_ws<double>(h, 6));
-  CHK(ensure_ws<T>(h, 7));
+  CHK(ensure_ws<T>(h, 2));
   double* r64 = h->w64[5];
-  T *r = h->w32[0], *xc = h->w32[1], *p = h->w32[2], *v = h->w32[3], *t = h->w32[4], *y = h->w32[5],
-    *rt = h->w32[6];
-  if (!h->d_bscal) HIPCHK(h, hipMalloc(&h->d_bscal, sizeof(double) * 8));
+  T *r = h->w32[0], *xc = h->w32[1];
+  BicgVecs<T> w;
+  CHK(bicg_vecs<T>(h, P, 2, xc, r, w));
   int* st = h->d_state;
   double* ds = h->d_dstate;
   double* bs = h->d_bscal;
-  A* part = partial_buf<A>(h);
-  const dim3 rg(kRedBlocks), rb(kRedThreads), fg(1), fb(kFinalThreads);
   auto residual64 = [&](double& d) -> int {
     CHK(apply64(h, x, r64, false, false));
     hipLaunchKernelGGL(axpy_kernel<double>, dim3(grid_for(n)), dim3(256), 0, h->stream, n, 1.0,
@@ -1173,21 +1254,9 @@ static int bicgstab_mixed_reliable(H* h, int precond, double inner_reduction, in
     HIPCHK(h, hipGetLastError());
     return PDELAB_OK;
   };
-  auto prec = [&](const T* in, T* out) -> int {
-    if (P.sor()) return sor_launch<T>(h, in, out, st, false);
-    if (P.ibj()) return ibj_launch<T>(h, in, out, static_cast<int*>(h->d_ibj_stat), nullptr, st, false);
-    if (P.block()) {
-      const BJVec<T, A> bv{in, out, nullptr, nullptr, nullptr, nullptr, st};
-      return bj_launch<T, A>(h, false, BJ_PREC, bv, nullptr);
-    }
-    hipLaunchKernelGGL(prec_stop_kernel<T>, dim3(grid_for(n)), dim3(256), 0, h->stream, n, P.dinv, in, out,
-                       (const int*)st);
-    HIPCHK(h, hipGetLastError());
-    return PDELAB_OK;
-  };
   // a fresh recurrence: rt = r, rho_new = rt.r, p = r at the first step
   auto start = [&]() -> int {
-    HIPCHK(h, hipMemcpyAsync(rt, r, sizeof(T) * n, hipMemcpyDeviceToDevice, h->stream));
+    HIPCHK(h, hipMemcpyAsync(w.rt, r, sizeof(T) * n, hipMemcpyDeviceToDevice, h->stream));
     CHK((dot_dev<T, A>(h, r, r, n, 0)));
     A sc[1];
     CHK((read_scalars<A>(h, sc, 1)));
@@ -1227,30 +1296,11 @@ static int bicgstab_mixed_reliable(H* h, int precond, double inner_reduction, in
         ++it;
         ++seg;
         if (!resume_second) {
-          hipLaunchKernelGGL(bicg_p_dev_kernel<T>, dim3(grid_for(n)), dim3(256), 0, h->stream, n, p, (const T*)r,
-                             (const T*)v, (const double*)bs, (const int*)st, first ? 1 : 0);
-          CHK(prec(p, y));
-          CHK(apply_mode<T>(h, y, v, false, 0, nullptr, st));
-          hipLaunchKernelGGL((dot_partial_kernel<T, A>), rg, rb, 0, h->stream, (const T*)rt, (const T*)v, n, part);
-          hipLaunchKernelGGL((bicg_scalar_kernel<A, 0>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                             2 * seg - 1);
-          hipLaunchKernelGGL((bicg_xr_kernel<T, A, 1>), rg, rb, 0, h->stream, n, xc, (const T*)y, r, (const T*)v,
-                             (const T*)nullptr, (const double*)bs, kBsAlpha, part, (const int*)st);
-          hipLaunchKernelGGL((bicg_scalar_kernel<A, 1>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                             2 * seg - 1);
+          CHK((bicg_first_half<T, A>(h, P, w, first, seg)));
           first = false;
         }
+        CHK((bicg_second_half<T, A>(h, P, w, resume_second, seg)));
         resume_second = false;
-        CHK(prec(r, y));
-        CHK(apply_mode<T>(h, y, t, false, 0, nullptr, st));
-        hipLaunchKernelGGL((dot2_kernel<T, A>), rg, rb, 0, h->stream, n, (const T*)t, (const T*)r, part);
-        hipLaunchKernelGGL((bicg_scalar_kernel<A, 2>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                           2 * seg);
-        hipLaunchKernelGGL((bicg_xr_kernel<T, A, 2>), rg, rb, 0, h->stream, n, xc, (const T*)y, r, (const T*)t,
-                           (const T*)rt, (const double*)bs, kBsOmega, part, (const int*)st);
-        hipLaunchKernelGGL((bicg_scalar_kernel<A, 3>), fg, fb, 0, h->stream, (const A*)part, kRedBlocks, bs, st, ds,
-                           2 * seg);
-        HIPCHK(h, hipGetLastError());
         if (seg % kBicgCheckEvery == 0 || it >= inner_maxit) {
           HIPCHK(h, hipMemcpyAsync(h->h_state, st, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
           HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -1292,7 +1342,7 @@ static int bicgstab_mixed_reliable(H* h, int precond, double inner_reduction, in
         continue;
       }
       // stopped after a full step: rho_new from the replaced residual, then beta
-      CHK((dot_dev<T, A>(h, rt, r, n, 0)));
+      CHK((dot_dev<T, A>(h, w.rt, r, n, 0)));
       A sc[1];
       CHK((read_scalars<A>(h, sc, 1)));
       double b[5];
@@ -1543,6 +1593,10 @@ int pdelab_gpu_synchronize(pdelab_gpu_gridoperator* h) {
 int pdelab_gpu_residual(pdelab_gpu_gridoperator* h, const double* x, double* r) {
   if (!h || !x || !r) return PDELAB_ERR_INVALID_ARG;
   CHK(compute_R0(h));
+  if (!h->varb && mfma_kernel(h)) {  // R(0) inside the apply: a pass of its own took 73 us at 64^3 Q3
+    CHK(check_outflow(h));
+    return launch_apply_mfma(h, x, r, false, 5, nullptr, nullptr, h->d_R0);
+  }
   CHK(apply64(h, x, r, false, true));
   hipLaunchKernelGGL(axpy_kernel<double>, dim3(grid_for(h->N)), dim3(256), 0, h->stream, h->N, 1.0,
                      (const double*)h->d_R0, r);

@@ -124,3 +124,50 @@ def test_mfma_velocity_edges(pkg, of, grid, kind, degree):
     yd.zero()
     go.jacobian_apply_transpose(zd, yd)
     assert np.linalg.norm(yd.download() - ref) <= RTOL * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("degree", [2, 3])
+@pytest.mark.parametrize("kind", ["const", "outflow", "cells", "cells_conv", "tensor"])
+@pytest.mark.parametrize("grid", GRIDS, ids=lambda g: "x".join(map(str, g)))
+def test_mfma_residual_edges(pkg, of, grid, kind, degree):
+    """r += R(x): R(0) is added by the apply. Tolerance RTOL of the apply's and the load's size."""
+    print(f"[gpu] matrix-core residual {grid} Q{degree} {kind}", flush=True)
+    nx, ny, nz = grid
+    cfg = pkg.make_config(nx=nx, ny=ny, nz=nz, degree=degree, alpha=3.0, problem=pkg.PROBLEM_CONSTANT, f0=1.0, **KINDS[kind])
+    rng = np.random.default_rng(11)
+    kappa = np.exp(rng.normal(size=pkg.ncells(cfg) * (3 if cfg.kappa_per_cell == 2 else 1))) if cfg.kappa_per_cell else None
+    go, o = pkg.GridOperator(cfg, kappa), of.Oracle(cfg, kappa)
+    x, r0 = rng.uniform(-1, 1, go.N), rng.uniform(-1, 1, go.N)
+    xd, rd = go.vector(x), go.vector(r0)
+    go.residual(xd, rd)
+    ref = o.residual(x)
+    assert np.linalg.norm(rd.download() - r0 - ref) <= RTOL * (np.linalg.norm(ref) + np.linalg.norm(r0))
+
+
+@pytest.mark.parametrize("precond", [0, 1, 2], ids=["none", "point", "block"])
+@pytest.mark.parametrize("degree", [1, 2, 3])
+@pytest.mark.parametrize("kind", ["const", "conv", "cells_conv", "tensor"])
+@pytest.mark.parametrize("grid", [(4, 1, 1), (5, 1, 2), (7, 5, 3), (13, 11, 35)], ids=lambda g: "x".join(map(str, g)))
+def test_bicgstab_first_iterations(pkg, of, grid, kind, degree, precond):
+    """The iterate after one and two BiCGSTAB iterations (Q1's dots are passes of their own, Q2's
+    and Q3's part of the apply), and the one at which a loose reduction stops, the half step
+    included. Two iterations form eight quotients of sums; each sum carries at most 1e-12 (the
+    apply's bound) times its cancellation, for which 1e4 is allowed: 1e-7 in all."""
+    print(f"[gpu] BiCGSTAB steps {grid} Q{degree} {kind} precond {precond}", flush=True)
+    nx, ny, nz = grid
+    cfg = pkg.make_config(nx=nx, ny=ny, nz=nz, degree=degree, alpha=3.0, **KINDS[kind])
+    rng = np.random.default_rng(13)
+    kappa = np.exp(rng.normal(size=pkg.ncells(cfg) * (3 if cfg.kappa_per_cell == 2 else 1))) if cfg.kappa_per_cell else None
+    go, o = pkg.GridOperator(cfg, kappa), of.Oracle(cfg, kappa)
+    b, x0 = rng.uniform(-1, 1, go.N), rng.uniform(-1, 1, go.N)
+    for maxit, reduction in ((1, 1e-14), (2, 1e-14), (50, 0.7), (50, 0.3)):
+        zd, rd = go.vector(x0), go.vector(b)
+        res = go.solve(zd, rd, method=pkg.SOLVER_BICGSTAB, precond=precond, reduction=reduction, maxit=maxit)
+        z_ref, _, ref = o.solve(b, x0, method=pkg.SOLVER_BICGSTAB, precond=precond, reduction=reduction, maxit=maxit)
+        if res["iterations"] > 2:
+            continue  # rounding has grown past what two iterations bound
+        assert res["iterations"] == ref["iterations"]
+        z, r = zd.download(), rd.download()
+        assert np.linalg.norm(z - z_ref) <= 1e-7 * np.linalg.norm(z_ref)
+        # the returned defect is that of the returned iterate
+        assert np.linalg.norm(r - (b - o.jacobian_apply(z))) <= 1e-10 * np.linalg.norm(b - o.jacobian_apply(x0))
