@@ -189,14 +189,56 @@ __global__ __launch_bounds__(kRedThreads) void prec_dot_kernel(long long n, cons
   if (threadIdx.x == 0) partial[blockIdx.x] = v[0];
 }
 
-// Device-side CG iteration (dune-istl CGSolver::apply, R:dune/istl/solvers.hh), five
-// launches per iteration: the apply with the fused p.q partials, their reduction into
-// scal[0] (cg_pq_kernel), cg_rupdate_kernel, cg_check_kernel and cg_xpupdate_kernel.
-// state = {stopped, aborted, stop iteration}; dstate = {defect, def0, reduction}. Every
-// kernel of an iteration after the one that stopped the loop returns at once.
+// Device-side CG iteration (dune-istl CGSolver::apply, R:dune/istl/solvers.hh): the apply with
+// the fused p.q partials, the update of r with the partials of (r.r, z.r), and the update of x
+// and p. The sums in between are finished by single-workgroup launches (cg_pq_kernel,
+// cg_check_kernel) or, where the partials are few, by every workgroup of the kernel that needs
+// them: a launch costs 3 to 6 us with its gap, summing a thousand partials in each of a
+// thousand workgroups 1 to 2 us. state = {iteration that stopped the loop or 0, aborted, iteration};
+// dstate = {defect, def0, reduction}. Every kernel of an iteration after the one that stopped
+// the loop returns at once.
 // Scalar slots of the step lengths: the single-workgroup kernels divide once, and the
 // vector kernels read the quotients (an FP64 division per wave cost ~10 us per launch).
 constexpr int kSlotLambda = 8, kSlotBeta = 9;
+
+// Most partials of one sum that the workgroups of a vector kernel add up themselves, and most
+// elements for which the x/p update does so: its grid is exact above, 65536 workgroups at 2^24.
+// us per iteration, point Jacobi, separate launches -> folded: 16^3 Q2 18.6 -> 13.1, 32^3 Q2 30.7 ->
+// 27.4, 48^3 Q2 71.5 -> 61.1, 64^3 Q2 (7.1M) 132.9 -> 122.8; 64^3 Q3 (16.8M) with only p.q folded
+// 306.3 -> 297.1, with the check folded too 307.3.
+constexpr int kFoldPartials = 2048;
+constexpr long long kFoldElements = 1LL << 23;
+
+// The sums of the partials, by every workgroup alike (kRedThreads threads): all threads of all
+// workgroups get the same bits.
+template <typename A, int NR>
+__device__ __forceinline__ void group_partial_sum(const A* __restrict__ partial, int nb, A (&v)[NR]) {
+  __shared__ A red[NR][kRedThreads / 64];
+#pragma unroll
+  for (int j = 0; j < NR; ++j) v[j] = A(0);
+  for (int b0 = threadIdx.x; b0 < nb; b0 += 4 * kRedThreads) {
+    A a[4][NR];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < NR; ++j) a[u][j] = b0 + u * kRedThreads < nb ? partial[(b0 + u * kRedThreads) * NR + j] : A(0);
+#pragma unroll
+    for (int j = 0; j < NR; ++j) v[j] += (a[0][j] + a[1][j]) + (a[2][j] + a[3][j]);
+  }
+#pragma unroll
+  for (int j = 0; j < NR; ++j) {
+    v[j] = wave_sum(v[j]);
+    if ((threadIdx.x & 63) == 0) red[j][threadIdx.x >> 6] = v[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NR; ++j) {
+    A s = red[j][0];
+#pragma unroll
+    for (int w = 1; w < kRedThreads / 64; ++w) s += red[j][w];
+    v[j] = s;
+  }
+}
 
 // scal[0] = p.q from the apply's partials, scal[kSlotLambda] = lambda = scal[slot_rho] / p.q
 template <typename A>
@@ -212,18 +254,19 @@ __global__ __launch_bounds__(kFinalThreads) void cg_pq_kernel(const A* __restric
   }
 }
 
-// r -= lambda q with lambda = scal[kSlotLambda]; partials of r.r and (dinv r).r
-template <typename T, typename A>
+// r -= lambda q; partials of r.r and (dinv r).r, two per workgroup. FOLD: lambda from the npq
+// partials of p.q at pq (and scal[0], scal[kSlotLambda] set, as cg_pq_kernel does), else from
+// scal[kSlotLambda].
+template <typename T, typename A, bool FOLD>
 __global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T* __restrict__ r, const T* __restrict__ q,
-                                                                 const T* __restrict__ dinv, const A* __restrict__ scal,
-                                                                 A* __restrict__ partial,
-                                                                 const int* __restrict__ state) {
+                                                                 const T* __restrict__ dinv, A* __restrict__ scal,
+                                                                 A* __restrict__ partial, const int* __restrict__ state,
+                                                                 const A* __restrict__ pq, int npq, int slot_rho) {
   if (state[0]) return;
-  const T lambda = (T)scal[kSlotLambda];
   A v[2] = {A(0), A(0)};
   const long long S = (long long)gridDim.x * kRedThreads;
-  for (long long i0 = (long long)blockIdx.x * kRedThreads + threadIdx.x; i0 < n; i0 += kVecUnroll * S) {
-    T rv[kVecUnroll], qv[kVecUnroll], dv[kVecUnroll];
+  T rv[kVecUnroll], qv[kVecUnroll], dv[kVecUnroll];
+  auto load = [&](long long i0) {
 #pragma unroll
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
@@ -235,6 +278,22 @@ __global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T*
         if (dinv) dv[u] = dinv[i];
       }
     }
+  };
+  const long long first = (long long)blockIdx.x * kRedThreads + threadIdx.x;
+  load(first);  // on their way while lambda is formed
+  T lambda;
+  if constexpr (FOLD) {
+    A s[1];
+    const A rho = scal[slot_rho];
+    group_partial_sum<A, 1>(pq, npq, s);
+    const A lam = rho / s[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      scal[0] = s[0];
+      scal[kSlotLambda] = lam;
+    }
+    lambda = (T)lam;
+  } else lambda = (T)scal[kSlotLambda];
+  for (long long i0 = first; i0 < n;) {
 #pragma unroll
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
@@ -246,6 +305,8 @@ __global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T*
         v[1] += (A)zi * (A)ri;
       }
     }
+    i0 += kVecUnroll * S;
+    if (i0 < n) load(i0);
   }
   block_sum_n<kRedThreads, A, 2>(v);
   if (threadIdx.x == 0) {
@@ -254,32 +315,34 @@ __global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T*
   }
 }
 
-// IterativeSolver::Iteration::step on the device (single workgroup): reduces the
-// partials of (r.r, z.r) into out[0..1], writes beta = z.r / rho_old (when beta is not
-// null), records the defect and the iteration number of a running loop and raises the
-// stop flag on convergence (def < reduction*def0 or def < 1e-30) or on a non-finite defect.
+// IterativeSolver::Iteration::step of iteration it: records the defect and the iteration and
+// raises the stop flag on convergence (def < reduction def0 or def < 1e-30) or on a non-finite
+// defect. `stops` is the decision alone.
+__device__ __forceinline__ bool cg_stops(double def, const double* __restrict__ dstate) {
+  return !isfinite(def) || def < dstate[1] * dstate[2] || def < 1e-30;
+}
+__device__ __forceinline__ void cg_record(double def, int it, int* __restrict__ state, double* __restrict__ dstate) {
+  state[2] = it;
+  dstate[0] = def;
+  if (!isfinite(def)) state[1] = 1;
+  if (cg_stops(def, dstate)) state[0] = it;
+}
+
+// The step on the device by one workgroup: reduces the partials of (r.r, z.r) into out[0..1] and
+// writes beta = z.r / rho_old.
 template <typename A>
 __global__ __launch_bounds__(kFinalThreads) void cg_check_kernel(const A* __restrict__ partial, int nb,
                                                                A* __restrict__ out, int* __restrict__ state,
                                                                double* __restrict__ dstate, int it,
-                                                               const A* __restrict__ rho_old = nullptr,
-                                                               A* __restrict__ beta = nullptr) {
+                                                               const A* __restrict__ rho_old, A* __restrict__ beta) {
   if (state[0]) return;
   A v[2];
   strided_partial_sum<A, 2>(partial, nb, v);
   if (threadIdx.x == 0) {
     out[0] = v[0];
     out[1] = v[1];
-    if (beta) *beta = v[1] / *rho_old;
-    const double def = sqrt((double)v[0]);
-    state[2] = it;
-    dstate[0] = def;
-    if (!isfinite(def)) {
-      state[1] = 1;
-      state[0] = 1;
-    } else if (def < dstate[1] * dstate[2] || def < 1e-30) {
-      state[0] = 1;
-    }
+    *beta = v[1] / *rho_old;
+    cg_record(sqrt((double)v[0]), it, state, dstate);
   }
 }
 
@@ -305,7 +368,7 @@ __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __rest
   // xp_ept<T>() contiguous elements per thread over an exact grid: the fastest of the
   // access patterns measured for this five-stream update
   constexpr int E = xp_ept<T>();
-  if (state[0] && state[2] < it) return;
+  if (state[0] && state[0] != it) return;
   const long long i0 = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * E;
   if (i0 >= n) return;
   const bool pupd = state[0] == 0;
@@ -343,6 +406,62 @@ __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __rest
         p[i] = zv + beta * pv;
       }
     }
+  }
+}
+
+// The same with the check of iteration `it` in front (cg_check_kernel's), by every workgroup from
+// the nparts pairs of partials: out[0..1] = (r.r, z.r), beta = z.r / *rho_old. Workgroup 0 records
+// the outcome; the others may see the flag it raises, so that the flag holds the iteration.
+template <typename T, typename A, int ZSRC>
+__global__ __launch_bounds__(kRedThreads) void cg_xpcheck_kernel(long long n, T* __restrict__ x, T* __restrict__ p,
+                                                                 const T* __restrict__ r, const T* __restrict__ dinv,
+                                                                 const T* __restrict__ z, const A* __restrict__ scal,
+                                                                 int* state, double* __restrict__ dstate, int it,
+                                                                 const A* __restrict__ partial, int nparts,
+                                                                 const A* __restrict__ rho_old, A* __restrict__ out) {
+  const int stopped = *(volatile int*)state;
+  if (stopped && stopped != it) return;
+  const long long S = (long long)gridDim.x * kRedThreads;
+  T xv[kVecUnroll], pv[kVecUnroll], zv[kVecUnroll];
+  auto load = [&](long long i0) {
+#pragma unroll
+    for (int u = 0; u < kVecUnroll; ++u) {
+      const long long i = i0 + u * S;
+      xv[u] = pv[u] = zv[u] = T(0);
+      if (i < n) {
+        xv[u] = x[i];
+        pv[u] = p[i];
+        if constexpr (ZSRC == XP_Z) zv[u] = z[i];
+        else if constexpr (ZSRC == XP_DINV_R) zv[u] = dinv[i] * r[i];
+        else zv[u] = r[i];
+      }
+    }
+  };
+  const long long first = (long long)blockIdx.x * kRedThreads + threadIdx.x;
+  load(first);  // on their way while the sums are formed
+  const T lambda = (T)scal[kSlotLambda];
+  const A rho = *rho_old;
+  A v[2];
+  group_partial_sum<A, 2>(partial, nparts, v);
+  const double def = sqrt((double)v[0]);
+  const T beta = (T)(v[1] / rho);
+  const bool pupd = !cg_stops(def, dstate);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    out[0] = v[0];
+    out[1] = v[1];
+    cg_record(def, it, state, dstate);
+  }
+  for (long long i0 = first; i0 < n;) {
+#pragma unroll
+    for (int u = 0; u < kVecUnroll; ++u) {
+      const long long i = i0 + u * S;
+      if (i < n) {
+        x[i] = xv[u] + lambda * pv[u];
+        if (pupd) p[i] = zv[u] + beta * pv[u];
+      }
+    }
+    i0 += kVecUnroll * S;
+    if (i0 < n) load(i0);
   }
 }
 

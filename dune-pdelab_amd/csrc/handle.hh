@@ -79,10 +79,11 @@ struct pdelab_gpu_gridoperator {
   double* h_scal64 = nullptr;
   float* h_scal32 = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  hipEvent_t evk[2] = {nullptr, nullptr};  // of the Krylov loop's copies of the state
   double* d_applydot = nullptr;  // per-workgroup partials of the fused apply dot
-  int* d_state = nullptr;        // device Krylov loop: {stopped, aborted, iteration, -}
+  int* d_state = nullptr;        // device Krylov loop: {stopped (CG: the iteration), aborted, iteration, -}
   double* d_dstate = nullptr;    // {defect, def0, reduction, -}
-  int* h_state = nullptr;        // pinned mirrors
+  int* h_state = nullptr;        // pinned mirrors (the state's twice)
   double* h_dstate = nullptr;
   double* d_bscal = nullptr;     // device BiCGSTAB loop: {rho, rho_new, alpha, omega, beta}
   DeviceTables* d_tab = nullptr;  // constants of the apply kernels

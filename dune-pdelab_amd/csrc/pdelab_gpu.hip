@@ -612,8 +612,9 @@ static int ensure_applydot(H* h) {
   return PDELAB_OK;
 }
 
-// Iterations between host reads of the device CG loop's stop flag.
-constexpr int kCheckEvery = 16;
+// Iterations between host reads of the device CG loop's stop flag, each of the state one such
+// interval earlier.
+constexpr int kCheckEvery = 8;
 
 // Outcome of one run of the device CG loop.
 struct CgLoopOut {
@@ -642,6 +643,9 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
   h->h_dstate[2] = red;
   HIPCHK(h, hipMemcpyAsync(h->d_state, h->h_state, sizeof(int) * 4, hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipMemcpyAsync(h->d_dstate, h->h_dstate, sizeof(double) * 4, hipMemcpyHostToDevice, h->stream));
+  // few partials: the vector kernels add them up themselves (blas_kernels.hh)
+  const bool fold_pq = !P.block() && nbapply <= kFoldPartials;
+  const int rblocks = (int)std::min<long long>(kRedBlocks, (n + 2 * kRedThreads - 1) / (2 * kRedThreads));
   bool stopped = false;
   int last = 0;
   for (int i = 1; i <= maxit && !stopped; ++i) {
@@ -650,40 +654,57 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
     // q = J p with the p.q partials -> scal[0]; r -= lambda q with the (r.r, z.r)
     // partials -> scal[oslot..] and the defect check; x += lambda p, p = z + beta p
     CHK(apply_mode<T>(h, p, q, trans, 2, dotp, h->d_state));
-    hipLaunchKernelGGL((cg_pq_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, (const A*)dotp, (int)nbapply,
-                       scal, rslot, (const int*)h->d_state);
+    if (!fold_pq)
+      hipLaunchKernelGGL((cg_pq_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, (const A*)dotp, (int)nbapply,
+                         scal, rslot, (const int*)h->d_state);
     const A* parts = partial_buf<A>(h);
-    int nparts = kRedBlocks;
+    int nparts = rblocks;
     if (P.block()) {
       // r -= lambda q and z = W^{-1} r in one pass over the cells (z is kept for the p update)
       const BJVec<T, A> v{b, z, b, q, scal + kSlotLambda, nullptr, h->d_state};
       CHK((bj_launch<T, A>(h, P.trans, BJ_CGR, v, &nparts)));
       parts = static_cast<const A*>(h->d_bjpart);
     } else {
-      hipLaunchKernelGGL((cg_rupdate_kernel<T, A>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, b,
-                         (const T*)q, P.dinv, (const A*)scal, partial_buf<A>(h), (const int*)h->d_state);
+      auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, b, (const T*)q, P.dinv, scal,
+                           partial_buf<A>(h), (const int*)h->d_state, (const A*)dotp, (int)nbapply, rslot);
+      };
+      if (fold_pq) run(cg_rupdate_kernel<T, A, true>);
+      else run(cg_rupdate_kernel<T, A, false>);
     }
-    hipLaunchKernelGGL((cg_check_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, parts, nparts, scal + oslot,
-                       h->d_state, h->d_dstate, i, (const A*)(scal + rslot), scal + kSlotBeta);
-    {
+    if (n <= kFoldElements && nparts <= kFoldPartials / 2) {
+      auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, x, p, (const T*)b, P.dinv,
+                           (const T*)z, (const A*)scal, h->d_state, h->d_dstate, i, parts, nparts,
+                           (const A*)(scal + rslot), scal + oslot);
+      };
+      if (P.block()) run(cg_xpcheck_kernel<T, A, XP_Z>);
+      else if (P.dinv) run(cg_xpcheck_kernel<T, A, XP_DINV_R>);
+      else run(cg_xpcheck_kernel<T, A, XP_R>);
+    } else {
+      hipLaunchKernelGGL((cg_check_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, parts, nparts, scal + oslot,
+                         h->d_state, h->d_dstate, i, (const A*)(scal + rslot), scal + kSlotBeta);
       const dim3 grid((unsigned)((n + 256LL * xp_ept<T>() - 1) / (256LL * xp_ept<T>())));
-      const T* zsrc = P.block() ? z : nullptr;
-      if (P.block())
-        hipLaunchKernelGGL((cg_xpupdate_kernel<T, A, XP_Z>), grid, dim3(256), 0, h->stream, n, x, p, (const T*)b, P.dinv,
-                           zsrc, (const A*)scal, (const int*)h->d_state, i);
-      else if (P.dinv)
-        hipLaunchKernelGGL((cg_xpupdate_kernel<T, A, XP_DINV_R>), grid, dim3(256), 0, h->stream, n, x, p, (const T*)b,
-                           P.dinv, zsrc, (const A*)scal, (const int*)h->d_state, i);
-      else
-        hipLaunchKernelGGL((cg_xpupdate_kernel<T, A, XP_R>), grid, dim3(256), 0, h->stream, n, x, p, (const T*)b, P.dinv,
-                           zsrc, (const A*)scal, (const int*)h->d_state, i);
+      auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, h->stream, n, x, p, (const T*)b, P.dinv, (const T*)z,
+                           (const A*)scal, (const int*)h->d_state, i);
+      };
+      if (P.block()) run(cg_xpupdate_kernel<T, A, XP_Z>);
+      else if (P.dinv) run(cg_xpupdate_kernel<T, A, XP_DINV_R>);
+      else run(cg_xpupdate_kernel<T, A, XP_R>);
     }
     HIPCHK(h, hipGetLastError());
     last = i;
+    // The flag is read while the next kCheckEvery iterations run: the stream never drains. What
+    // was enqueued after the stop returns at once.
     if (i % kCheckEvery == 0 || i == maxit) {
-      HIPCHK(h, hipMemcpyAsync(h->h_state, h->d_state, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
-      HIPCHK(h, hipStreamSynchronize(h->stream));
-      stopped = h->h_state[0] != 0;
+      const int k = i / kCheckEvery & 1;
+      HIPCHK(h, hipMemcpyAsync(h->h_state + 4 * k, h->d_state, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
+      HIPCHK(h, hipEventRecord(h->evk[k], h->stream));
+      if (i > kCheckEvery) {
+        HIPCHK(h, hipEventSynchronize(h->evk[k ^ 1]));
+        stopped = h->h_state[4 * (k ^ 1)] != 0;
+      }
     }
   }
   HIPCHK(h, hipMemcpyAsync(h->h_state, h->d_state, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
@@ -1438,9 +1459,11 @@ int pdelab_gpu_create(const pdelab_config* cfg, const double* kappa_host, pdelab
   if (hipHostMalloc(&h->h_scal64, sizeof(double) * 16) != hipSuccess) return bail("hipHostMalloc failed");
   if (hipHostMalloc(&h->h_scal32, sizeof(float) * 16) != hipSuccess) return bail("hipHostMalloc failed");
   if (hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess) return bail("hipEventCreate failed");
+  for (hipEvent_t& e : h->evk)
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return bail("hipEventCreate failed");
   if (hipMalloc(&h->d_state, sizeof(int) * 4) != hipSuccess) return bail("hipMalloc failed");
   if (hipMalloc(&h->d_dstate, sizeof(double) * 4) != hipSuccess) return bail("hipMalloc failed");
-  if (hipHostMalloc(&h->h_state, sizeof(int) * 4) != hipSuccess) return bail("hipHostMalloc failed");
+  if (hipHostMalloc(&h->h_state, sizeof(int) * 8) != hipSuccess) return bail("hipHostMalloc failed");
   if (hipHostMalloc(&h->h_dstate, sizeof(double) * 4) != hipSuccess) return bail("hipHostMalloc failed");
   if (init_scratch(h) != PDELAB_OK) return bail(h->err);
   if (cfg->kappa_per_cell) {
@@ -1478,6 +1501,8 @@ int pdelab_gpu_destroy(pdelab_gpu_gridoperator* h) {
   if (h->h_state) (void)hipHostFree(h->h_state);
   if (h->h_dstate) (void)hipHostFree(h->h_dstate);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
+  for (hipEvent_t e : h->evk)
+    if (e) (void)hipEventDestroy(e);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
