@@ -29,7 +29,7 @@
 
 namespace pdelab_amd {
 
-enum { BJ_PREC = 0, BJ_ADD = 1, BJ_CGR = 2 };
+enum { BJ_PREC = 0, BJ_ADD = 1, BJ_CGR = 2, BJ_CGD = 3, BJ_CGX = 4 };
 
 __host__ __device__ inline int bj_type(int i, int n) { return (i == 0 ? 1 : 0) | (i == n - 1 ? 2 : 0); }
 
@@ -443,6 +443,12 @@ __global__ __launch_bounds__(256) void bj_dense_setup_kernel(const DGArgs<double
 //   BJ_ADD : out += W^{-1} in
 //   BJ_CGR : r -= lambda q (lambda = *lam), out = W^{-1} r, partials
 //            of (r.r, out.r) per workgroup
+//   BJ_CGD : the same without out; BJ_CGX: x += lambda p, p = W^{-1} in + beta p. Fast
+//            diagonalisation by boundary type only, whose data stay in LDS: W^{-1} r is applied a
+//            second time instead of written and read back, and the dot needs its forward half only
+//            (64^3 Q3, 134 MB per vector: 8 instead of 9 streams, 83 + 101 -> 63 + 95 us, 6.5 and
+//            7.1 TB/s, and the apply that follows finds more of p in the cache, 70 -> 50 us). Vectors
+//            of up to 2^23 elements take BJ_CGR: their p update has the check in it
 // Every mode returns at once when a state is given and its stop flag state[0] is set (the
 // device-side Krylov loops).
 template <typename T, typename A>
@@ -454,6 +460,9 @@ struct BJVec {
   const A* lam;
   A* partial;
   const int* state;
+  T *x, *p;  // BJ_CGX: iterate and direction, beta, the CG iteration
+  const A* beta;
+  int it;
 };
 
 // Orders the LDS accesses of one wave (the wave executes them in program order; the
@@ -687,7 +696,9 @@ __global__ __launch_bounds__(BJFdmShape<N1>::THREADS) void bj_fdm_kernel(const B
                                                                         const T* __restrict__ data, const BJGeom g) {
   using S = BJFdmShape<N1>;
   constexpr int NL = S::NL, LPC = S::LPC, CPW = S::CPW, ES = S::ES;
-  if (v.state && v.state[0]) return;  // a device-side Krylov loop has already stopped
+  constexpr bool CGR = MODE == BJ_CGR || MODE == BJ_CGD;
+  // a device-side Krylov loop has already stopped (BJ_CGX: before this iteration)
+  if (v.state && v.state[0] && (MODE != BJ_CGX || v.state[0] != v.it)) return;
   // lines of the wave's cells, value k of lane l at X[w][k][l]: the sweep reads of a wave
   // touch every LDS bank at most twice (64-bit) or once (32-bit)
   __shared__ T X[S::WAVES][N1][64];
@@ -720,20 +731,24 @@ __global__ __launch_bounds__(BJFdmShape<N1>::THREADS) void bj_fdm_kernel(const B
     __syncthreads();
   }
   T lambda = T(0);
-  if (MODE == BJ_CGR) lambda = (T)*v.lam;
+  if (CGR || MODE == BJ_CGX) lambda = (T)*v.lam;
   A acc0 = A(0);
-  T u[N1];
+  T u[N1], xv[MODE == BJ_CGX ? N1 : 1], pv[MODE == BJ_CGX ? N1 : 1];
 #pragma unroll
   for (int k = 0; k < N1; ++k) {
     u[k] = T(0);
     if (act) {
       const long long idx = base + LPC * k;
-      if (MODE == BJ_CGR) {
+      if constexpr (CGR) {
         // r (reread next iteration) and q (dead after this step) stream past the caches
         const T x = ld_stream<T>(v.in + idx) - lambda * ld_stream<T>(v.q + idx);
         st_stream<T>(x, v.r + idx);
         acc0 += (A)x * (A)x;
         u[k] = x;
+      } else if constexpr (MODE == BJ_CGX) {
+        u[k] = ld_stream<T>(v.in + idx);
+        xv[k] = ld_stream<T>(v.x + idx);
+        pv[k] = v.p[idx];
       } else {
         u[k] = v.in[idx];
       }
@@ -808,6 +823,7 @@ __global__ __launch_bounds__(BJFdmShape<N1>::THREADS) void bj_fdm_kernel(const B
     t[k] = s * bj_rcp(lxy + lz[k]);
     dot += (A)s * (A)t[k];
   }
+  if constexpr (MODE != BJ_CGD) {  // the dot above needs no backward sweep
 #pragma unroll
   for (int k = 0; k < N1; ++k) {
     T s = T(0);
@@ -841,20 +857,26 @@ __global__ __launch_bounds__(BJFdmShape<N1>::THREADS) void bj_fdm_kernel(const B
   for (int m = 0; m < N1; ++m)
 #pragma unroll
     for (int k = 0; k < N1; ++k) u[k] += cf[m] * X[w][k][xo + m + N1 * iy];
+  const bool pupd = MODE == BJ_CGX && v.state[0] == 0;  // on the iteration that stopped the loop only x
+  const T beta = pupd ? (T)*v.beta : T(0);
   if (act) {
 #pragma unroll
     for (int k = 0; k < N1; ++k) {
       const long long idx = base + LPC * k;
-      if (MODE == BJ_ADD) v.out[idx] += u[k];
+      if constexpr (MODE == BJ_CGX) {
+        st_stream<T>(xv[k] + lambda * pv[k], v.x + idx);
+        if (pupd) v.p[idx] = u[k] + beta * pv[k];
+      } else if (MODE == BJ_ADD) v.out[idx] += u[k];
       else v.out[idx] = u[k];
     }
   }
-  if (MODE == BJ_PREC || MODE == BJ_CGR) {
-    // out.in (for BJ_CGR out.r with the updated r) from the active lanes only: a lane
+  }
+  if (MODE == BJ_PREC || CGR) {
+    // out.in (for BJ_CGR and BJ_CGD W^{-1} r.r with the updated r) from the active lanes only: a lane
     // beyond the wave's cells (lane 63 at Q2) aliases cell 0 in the sweeps and holds its
     // transformed values, which must not be counted twice
     const A d = act ? dot : A(0);
-    // one partial (BJ_PREC) or pair (BJ_CGR) per workgroup, reduced through X
+    // one partial (BJ_PREC) or pair (BJ_CGR, BJ_CGD) per workgroup, reduced through X
     if (MODE == BJ_PREC) {
       A r[1] = {d};
       block_sum_reuse<S::WAVES, A, 1>(r, &X[0][0][0]);

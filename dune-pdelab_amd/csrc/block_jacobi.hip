@@ -157,7 +157,14 @@ template <int N1, typename T, typename A, int MODE>
 int launch_n(H* h, const BlockJacobiData& b, const T* data, const BJVec<T, A>& v) {
   const BJGeom g = geom(h, b.per_cell);
   const long long nb = bj_groups(h, b.fdm);
-  if (b.fdm && b.per_cell)
+  if constexpr (MODE == BJ_CGD || MODE == BJ_CGX) {  // bj_cg_recompute() holds
+    if (((long long)g.n[0] * g.n[1]) % BJFdmShape<N1>::CPW == 0)
+      hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, false, true>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0,
+                         h->stream, v, data, g);
+    else
+      hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, false>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0, h->stream,
+                         v, data, g);
+  } else if (b.fdm && b.per_cell)
     hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, true>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0, h->stream, v,
                        data, g);
   else if (b.fdm && ((long long)g.n[0] * g.n[1]) % BJFdmShape<N1>::CPW == 0)
@@ -285,7 +292,14 @@ int bj_launch(H* h, bool trans, int mode, BJVec<T, A> v, int* nparts) {
   if (nparts) *nparts = (int)bj_partials(h, b);
   if (mode == BJ_PREC) return launch_m<T, A, BJ_PREC>(h, b, data, v);
   if (mode == BJ_ADD) return launch_m<T, A, BJ_ADD>(h, b, data, v);
+  if (mode == BJ_CGD) return launch_m<T, A, BJ_CGD>(h, b, data, v);
+  if (mode == BJ_CGX) return launch_m<T, A, BJ_CGX>(h, b, data, v);
   return launch_m<T, A, BJ_CGR>(h, b, data, v);
+}
+
+bool bj_cg_recompute(const H* h, bool trans) {
+  const BlockJacobiData& b = h->bj[trans ? 1 : 0];
+  return b.fdm && !b.per_cell;
 }
 
 template int bj_launch<double, double>(H*, bool, int, BJVec<double, double>, int*);

@@ -278,7 +278,7 @@ int mfma_vel_setup(H* h);
 int mfma_weights(H* h);  // d_fw64 from the current face coefficients
 
 // Block Jacobi (block_jacobi.hip): data set-up for the given precision (64 or 32),
-// invalidation when kappa changes, the launches (BJ_PREC / BJ_ADD / BJ_CGR, see
+// invalidation when kappa changes, the launches (BJ_PREC / BJ_ADD / BJ_CGR / BJ_CGD / BJ_CGX, see
 // block_jacobi.hh; the partials go to d_bjpart, their count to *nparts) and the
 // diagonal blocks themselves (ncells * nloc^2, row-major).
 int bj_prepare(H* h, bool trans, int precision);
@@ -286,6 +286,8 @@ void bj_invalidate(H* h);
 void bj_free(H* h);
 template <typename T, typename A>
 int bj_launch(H* h, bool trans, int mode, BJVec<T, A> v, int* nparts);
+// Whether the CG loop lets the p update apply W^{-1} again (BJ_CGD, BJ_CGX) instead of storing z.
+bool bj_cg_recompute(const H* h, bool trans);
 int bj_block_diagonal(H* h, bool trans, double* blocks);
 // Block SOR (block_sor.hh): data set-up (dense blocks of J) and one sweep, from v = 0
 // (v = W^{-1} d, the solvers) or in place from the v given (inplace); the kernels store

@@ -645,6 +645,8 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
   HIPCHK(h, hipMemcpyAsync(h->d_dstate, h->h_dstate, sizeof(double) * 4, hipMemcpyHostToDevice, h->stream));
   // few partials: the vector kernels add them up themselves (blas_kernels.hh)
   const bool fold_pq = !P.block() && nbapply <= kFoldPartials;
+  const bool fold_check = n <= kFoldElements;  // and few enough of them
+  const bool recompute = P.block() && !fold_check && bj_cg_recompute(h, P.trans);
   const int rblocks = (int)std::min<long long>(kRedBlocks, (n + 2 * kRedThreads - 1) / (2 * kRedThreads));
   bool stopped = false;
   int last = 0;
@@ -660,9 +662,10 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
     const A* parts = partial_buf<A>(h);
     int nparts = rblocks;
     if (P.block()) {
-      // r -= lambda q and z = W^{-1} r in one pass over the cells (z is kept for the p update)
+      // r -= lambda q and z = W^{-1} r in one pass over the cells (z is kept for the p update,
+      // or formed again there)
       const BJVec<T, A> v{b, z, b, q, scal + kSlotLambda, nullptr, h->d_state};
-      CHK((bj_launch<T, A>(h, P.trans, BJ_CGR, v, &nparts)));
+      CHK((bj_launch<T, A>(h, P.trans, recompute ? BJ_CGD : BJ_CGR, v, &nparts)));
       parts = static_cast<const A*>(h->d_bjpart);
     } else {
       auto run = [&](auto kernel) {
@@ -672,7 +675,7 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
       if (fold_pq) run(cg_rupdate_kernel<T, A, true>);
       else run(cg_rupdate_kernel<T, A, false>);
     }
-    if (n <= kFoldElements && nparts <= kFoldPartials / 2) {
+    if (fold_check && nparts <= kFoldPartials / 2) {
       auto run = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, x, p, (const T*)b, P.dinv,
                            (const T*)z, (const A*)scal, h->d_state, h->d_dstate, i, parts, nparts,
@@ -689,7 +692,10 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
         hipLaunchKernelGGL(kernel, grid, dim3(256), 0, h->stream, n, x, p, (const T*)b, P.dinv, (const T*)z,
                            (const A*)scal, (const int*)h->d_state, i);
       };
-      if (P.block()) run(cg_xpupdate_kernel<T, A, XP_Z>);
+      if (recompute) {
+        const BJVec<T, A> v{b, nullptr, nullptr, nullptr, scal + kSlotLambda, nullptr, h->d_state, x, p, scal + kSlotBeta, i};
+        CHK((bj_launch<T, A>(h, P.trans, BJ_CGX, v, nullptr)));
+      } else if (P.block()) run(cg_xpupdate_kernel<T, A, XP_Z>);
       else if (P.dinv) run(cg_xpupdate_kernel<T, A, XP_DINV_R>);
       else run(cg_xpupdate_kernel<T, A, XP_R>);
     }

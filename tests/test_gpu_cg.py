@@ -2,7 +2,7 @@
 preconditioner of the library's own (elsewhere tested) entry points: the iterate and the defect
 after a few iterations and at a loose reduction. The sizes are those where the loop's kernels
 change: vectors shorter than a workgroup, sums finished by the vector kernels or by launches of
-their own (2048 partials, 2^23 elements).
+their own (2048 partials, 2^23 elements), block Jacobi applied again instead of stored.
 
 Tolerance: three iterations form six quotients of sums; each sum carries at most 1e-12 (the
 apply's bound) times its cancellation, for which 1e4 is allowed: 1e-7 in all.
