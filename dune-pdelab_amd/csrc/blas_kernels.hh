@@ -254,26 +254,29 @@ __global__ __launch_bounds__(kFinalThreads) void cg_pq_kernel(const A* __restric
   }
 }
 
-// r -= lambda q; partials of r.r and (dinv r).r, two per workgroup. FOLD: lambda from the npq
+// z = W^{-1} r: z -= lambda dinv q (r -= lambda q without a preconditioner); partials of r.r and
+// z.r with r = z / dinv, two per workgroup. The loop carries z in r's place, so that the x/p update
+// reads one vector, not r and dinv: FP32 64^3 Q3 (67 MB per vector) x/p 57.9 -> 51.3 us, this kernel
+// 39.1 -> 39.5 us; FP64 CG at 64^3 Q3 297 -> 276 us per iteration. FOLD: lambda from the npq
 // partials of p.q at pq (and scal[0], scal[kSlotLambda] set, as cg_pq_kernel does), else from
 // scal[kSlotLambda].
 template <typename T, typename A, bool FOLD>
-__global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T* __restrict__ r, const T* __restrict__ q,
+__global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T* __restrict__ z, const T* __restrict__ q,
                                                                  const T* __restrict__ dinv, A* __restrict__ scal,
                                                                  A* __restrict__ partial, const int* __restrict__ state,
                                                                  const A* __restrict__ pq, int npq, int slot_rho) {
   if (state[0]) return;
   A v[2] = {A(0), A(0)};
   const long long S = (long long)gridDim.x * kRedThreads;
-  T rv[kVecUnroll], qv[kVecUnroll], dv[kVecUnroll];
+  T zv[kVecUnroll], qv[kVecUnroll], dv[kVecUnroll];
   auto load = [&](long long i0) {
 #pragma unroll
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
-      rv[u] = qv[u] = T(0);
+      zv[u] = qv[u] = T(0);
       dv[u] = T(1);
-      if (i < n) {  // r and q stream in; r is stored cached for the x/p update that follows
-        rv[u] = ld_stream<T>(r + i);
+      if (i < n) {  // z and q stream in; z is stored cached for the x/p update that follows
+        zv[u] = ld_stream<T>(z + i);
         qv[u] = ld_stream<T>(q + i);
         if (dinv) dv[u] = dinv[i];
       }
@@ -298,9 +301,9 @@ __global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T*
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
       if (i < n) {
-        const T ri = rv[u] - lambda * qv[u];
-        r[i] = ri;
-        const T zi = dv[u] * ri;
+        const T zi = zv[u] - lambda * (dv[u] * qv[u]);
+        z[i] = zi;
+        const T ri = dinv ? zi / dv[u] : zi;
         v[0] += (A)ri * (A)ri;
         v[1] += (A)zi * (A)ri;
       }
@@ -346,23 +349,16 @@ __global__ __launch_bounds__(kFinalThreads) void cg_check_kernel(const A* __rest
   }
 }
 
-// x += lambda p (lambda = scal[kSlotLambda]), then p = z + beta p with
-// beta = scal[kSlotBeta] and z = W^{-1} r: the given z (block Jacobi), else
-// dinv r or r; on the iteration that stopped the loop only x is updated (dune-istl leaves
-// the loop after the defect check).
+// x += lambda p (lambda = scal[kSlotLambda]), then p = z + beta p with beta = scal[kSlotBeta]; on
+// the iteration that stopped the loop only x is updated (dune-istl leaves the loop after the
+// defect check).
 // Elements per thread of the x/p update: one double, or two contiguous floats (8 B per
 // lane and stream either way).
 template <typename T>
 constexpr int xp_ept() { return sizeof(T) == 4 ? 2 : 1; }
 
-// Source of z: the given vector (block Jacobi), dinv r (point Jacobi) or r (none), fixed at
-// compile time (alone at 2^24 doubles the run-time choice cost 104.5 against 96.8 us; inside
-// the CG loop the two are within noise).
-enum { XP_Z = 0, XP_DINV_R = 1, XP_R = 2 };
-
-template <typename T, typename A, int ZSRC>
+template <typename T, typename A>
 __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __restrict__ x, T* __restrict__ p,
-                                                          const T* __restrict__ r, const T* __restrict__ dinv,
                                                           const T* __restrict__ z, const A* __restrict__ scal,
                                                           const int* __restrict__ state, int it) {
   // xp_ept<T>() contiguous elements per thread over an exact grid: the fastest of the
@@ -374,21 +370,14 @@ __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __rest
   const bool pupd = state[0] == 0;
   const T lambda = (T)scal[kSlotLambda];
   const T beta = pupd ? (T)scal[kSlotBeta] : T(0);
-  // x and z (or r) stream (non-temporal); p, reread by the next apply, stays cached
+  // x and z stream (non-temporal); p, reread by the next apply, stays cached
   if constexpr (E == 2) {
     if (i0 + 1 < n) {  // two contiguous floats as one 8-byte access per stream
       typedef T v2 __attribute__((ext_vector_type(2)));
       const v2 pv = *reinterpret_cast<const v2*>(p + i0);
       v2* xv = reinterpret_cast<v2*>(x + i0);
       st_stream<v2>(ld_stream<v2>(xv) + lambda * pv, xv);
-      if (pupd) {
-        v2 zv;
-        if constexpr (ZSRC == XP_Z) zv = ld_stream<v2>(reinterpret_cast<const v2*>(z + i0));
-        else if constexpr (ZSRC == XP_DINV_R)
-          zv = *reinterpret_cast<const v2*>(dinv + i0) * ld_stream<v2>(reinterpret_cast<const v2*>(r + i0));
-        else zv = ld_stream<v2>(reinterpret_cast<const v2*>(r + i0));
-        *reinterpret_cast<v2*>(p + i0) = zv + beta * pv;
-      }
+      if (pupd) *reinterpret_cast<v2*>(p + i0) = ld_stream<v2>(reinterpret_cast<const v2*>(z + i0)) + beta * pv;
       return;
     }
   }
@@ -398,23 +387,23 @@ __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __rest
     if (i < n) {
       const T pv = p[i];
       st_stream<T>(ld_stream<T>(x + i) + lambda * pv, x + i);
-      if (pupd) {
-        T zv;
-        if constexpr (ZSRC == XP_Z) zv = ld_stream<T>(z + i);
-        else if constexpr (ZSRC == XP_DINV_R) zv = dinv[i] * ld_stream<T>(r + i);
-        else zv = ld_stream<T>(r + i);
-        p[i] = zv + beta * pv;
-      }
+      if (pupd) p[i] = ld_stream<T>(z + i) + beta * pv;
     }
   }
+}
+
+// b *= d or b /= d: between r and z = W^{-1} r = dinv r at the ends of the loop
+template <typename T, bool DIV>
+__global__ __launch_bounds__(256) void cg_scale_kernel(long long n, T* __restrict__ b, const T* __restrict__ d) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    b[i] = DIV ? b[i] / d[i] : b[i] * d[i];
 }
 
 // The same with the check of iteration `it` in front (cg_check_kernel's), by every workgroup from
 // the nparts pairs of partials: out[0..1] = (r.r, z.r), beta = z.r / *rho_old. Workgroup 0 records
 // the outcome; the others may see the flag it raises, so that the flag holds the iteration.
-template <typename T, typename A, int ZSRC>
+template <typename T, typename A>
 __global__ __launch_bounds__(kRedThreads) void cg_xpcheck_kernel(long long n, T* __restrict__ x, T* __restrict__ p,
-                                                                 const T* __restrict__ r, const T* __restrict__ dinv,
                                                                  const T* __restrict__ z, const A* __restrict__ scal,
                                                                  int* state, double* __restrict__ dstate, int it,
                                                                  const A* __restrict__ partial, int nparts,
@@ -431,9 +420,7 @@ __global__ __launch_bounds__(kRedThreads) void cg_xpcheck_kernel(long long n, T*
       if (i < n) {
         xv[u] = x[i];
         pv[u] = p[i];
-        if constexpr (ZSRC == XP_Z) zv[u] = z[i];
-        else if constexpr (ZSRC == XP_DINV_R) zv[u] = dinv[i] * r[i];
-        else zv[u] = r[i];
+        zv[u] = z[i];
       }
     }
   };

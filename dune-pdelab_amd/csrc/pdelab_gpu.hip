@@ -648,12 +648,16 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
   const bool fold_check = n <= kFoldElements;  // and few enough of them
   const bool recompute = P.block() && !fold_check && bj_cg_recompute(h, P.trans);
   const int rblocks = (int)std::min<long long>(kRedBlocks, (n + 2 * kRedThreads - 1) / (2 * kRedThreads));
+  // point Jacobi: z = dinv r in b's place until the loop ends
+  const T* zv = P.block() ? z : b;
+  if (P.dinv)
+    hipLaunchKernelGGL((cg_scale_kernel<T, false>), dim3(grid_for(n)), dim3(256), 0, h->stream, n, b, P.dinv);
   bool stopped = false;
   int last = 0;
   for (int i = 1; i <= maxit && !stopped; ++i) {
     const int rslot = (i & 1) ? 7 : 5;  // slot holding the current rho
     const int oslot = (i & 1) ? 4 : 6;  // (def^2, rho_new) written here
-    // q = J p with the p.q partials -> scal[0]; r -= lambda q with the (r.r, z.r)
+    // q = J p with the p.q partials -> scal[0]; r -= lambda q (as z) with the (r.r, z.r)
     // partials -> scal[oslot..] and the defect check; x += lambda p, p = z + beta p
     CHK(apply_mode<T>(h, p, q, trans, 2, dotp, h->d_state));
     if (!fold_pq)
@@ -676,28 +680,20 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
       else run(cg_rupdate_kernel<T, A, false>);
     }
     if (fold_check && nparts <= kFoldPartials / 2) {
-      auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, x, p, (const T*)b, P.dinv,
-                           (const T*)z, (const A*)scal, h->d_state, h->d_dstate, i, parts, nparts,
-                           (const A*)(scal + rslot), scal + oslot);
-      };
-      if (P.block()) run(cg_xpcheck_kernel<T, A, XP_Z>);
-      else if (P.dinv) run(cg_xpcheck_kernel<T, A, XP_DINV_R>);
-      else run(cg_xpcheck_kernel<T, A, XP_R>);
+      hipLaunchKernelGGL((cg_xpcheck_kernel<T, A>), dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, x, p, zv,
+                         (const A*)scal, h->d_state, h->d_dstate, i, parts, nparts, (const A*)(scal + rslot),
+                         scal + oslot);
     } else {
       hipLaunchKernelGGL((cg_check_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, parts, nparts, scal + oslot,
                          h->d_state, h->d_dstate, i, (const A*)(scal + rslot), scal + kSlotBeta);
-      const dim3 grid((unsigned)((n + 256LL * xp_ept<T>() - 1) / (256LL * xp_ept<T>())));
-      auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, h->stream, n, x, p, (const T*)b, P.dinv, (const T*)z,
-                           (const A*)scal, (const int*)h->d_state, i);
-      };
       if (recompute) {
         const BJVec<T, A> v{b, nullptr, nullptr, nullptr, scal + kSlotLambda, nullptr, h->d_state, x, p, scal + kSlotBeta, i};
         CHK((bj_launch<T, A>(h, P.trans, BJ_CGX, v, nullptr)));
-      } else if (P.block()) run(cg_xpupdate_kernel<T, A, XP_Z>);
-      else if (P.dinv) run(cg_xpupdate_kernel<T, A, XP_DINV_R>);
-      else run(cg_xpupdate_kernel<T, A, XP_R>);
+      } else {
+        const dim3 grid((unsigned)((n + 256LL * xp_ept<T>() - 1) / (256LL * xp_ept<T>())));
+        hipLaunchKernelGGL((cg_xpupdate_kernel<T, A>), grid, dim3(256), 0, h->stream, n, x, p, zv, (const A*)scal,
+                           (const int*)h->d_state, i);
+      }
     }
     HIPCHK(h, hipGetLastError());
     last = i;
@@ -713,6 +709,8 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
       }
     }
   }
+  if (P.dinv)
+    hipLaunchKernelGGL((cg_scale_kernel<T, true>), dim3(grid_for(n)), dim3(256), 0, h->stream, n, b, P.dinv);
   HIPCHK(h, hipMemcpyAsync(h->h_state, h->d_state, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipMemcpyAsync(h->h_dstate, h->d_dstate, sizeof(double) * 4, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
