@@ -254,13 +254,29 @@ __global__ __launch_bounds__(kFinalThreads) void cg_pq_kernel(const A* __restric
   }
 }
 
+// Which of an iteration's vectors are left in the 256 MB memory-side cache. x and dinv are read once
+// and stream past it unless all five fit; p, q and z, which the next kernels read again, stay while
+// these three fit; else only p, for the apply. Mixed solve at 64^3 Q3 lognormal (67 MB per vector):
+// z and q streamed, dinv cached 519 ms, z and q kept, dinv streamed 505 ms, dinv cached as well 535 ms.
+// FP64 CG at 64^3 Q3 (134 MB): dinv cached 829 ms, streamed 766 ms; with z and q kept 839 ms. At 72^3 Q2
+// (81 MB) 281, 273 and 290 ms. Mixed solve at 64^3 Q2 (28 MB): all cached 152 ms, as before 157 ms.
+enum { CG_STREAM = 0, CG_KEEP = 1, CG_ALL = 2 };
+constexpr int cg_cache(long long bytes) {
+  return 5 * bytes <= 224LL << 20 ? CG_ALL : (3 * bytes <= 224LL << 20 ? CG_KEEP : CG_STREAM);
+}
+template <bool STREAM, typename V>
+__device__ __forceinline__ V ld_vec(const V* p) {
+  if constexpr (STREAM) return ld_stream<V>(p);
+  else return *p;
+}
+
 // z = W^{-1} r: z -= lambda dinv q (r -= lambda q without a preconditioner); partials of r.r and
 // z.r with r = z / dinv, two per workgroup. The loop carries z in r's place, so that the x/p update
 // reads one vector, not r and dinv: FP32 64^3 Q3 (67 MB per vector) x/p 57.9 -> 51.3 us, this kernel
 // 39.1 -> 39.5 us; FP64 CG at 64^3 Q3 297 -> 276 us per iteration. FOLD: lambda from the npq
 // partials of p.q at pq (and scal[0], scal[kSlotLambda] set, as cg_pq_kernel does), else from
 // scal[kSlotLambda].
-template <typename T, typename A, bool FOLD>
+template <typename T, typename A, bool FOLD, int CACHE>
 __global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T* __restrict__ z, const T* __restrict__ q,
                                                                  const T* __restrict__ dinv, A* __restrict__ scal,
                                                                  A* __restrict__ partial, const int* __restrict__ state,
@@ -275,10 +291,10 @@ __global__ __launch_bounds__(kRedThreads) void cg_rupdate_kernel(long long n, T*
       const long long i = i0 + u * S;
       zv[u] = qv[u] = T(0);
       dv[u] = T(1);
-      if (i < n) {  // z and q stream in; z is stored cached for the x/p update that follows
-        zv[u] = ld_stream<T>(z + i);
-        qv[u] = ld_stream<T>(q + i);
-        if (dinv) dv[u] = dinv[i];
+      if (i < n) {  // z is stored cached for the x/p update that follows
+        zv[u] = ld_vec<CACHE == CG_STREAM>(z + i);
+        qv[u] = ld_vec<CACHE == CG_STREAM>(q + i);
+        if (dinv) dv[u] = ld_vec<CACHE != CG_ALL>(dinv + i);
       }
     }
   };
@@ -357,7 +373,7 @@ __global__ __launch_bounds__(kFinalThreads) void cg_check_kernel(const A* __rest
 template <typename T>
 constexpr int xp_ept() { return sizeof(T) == 4 ? 2 : 1; }
 
-template <typename T, typename A>
+template <typename T, typename A, bool KEEP>
 __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __restrict__ x, T* __restrict__ p,
                                                           const T* __restrict__ z, const A* __restrict__ scal,
                                                           const int* __restrict__ state, int it) {
@@ -370,14 +386,14 @@ __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __rest
   const bool pupd = state[0] == 0;
   const T lambda = (T)scal[kSlotLambda];
   const T beta = pupd ? (T)scal[kSlotBeta] : T(0);
-  // x and z stream (non-temporal); p, reread by the next apply, stays cached
+  // x streams (non-temporal); p, reread by the next apply, stays cached, z if KEEP
   if constexpr (E == 2) {
     if (i0 + 1 < n) {  // two contiguous floats as one 8-byte access per stream
       typedef T v2 __attribute__((ext_vector_type(2)));
       const v2 pv = *reinterpret_cast<const v2*>(p + i0);
       v2* xv = reinterpret_cast<v2*>(x + i0);
       st_stream<v2>(ld_stream<v2>(xv) + lambda * pv, xv);
-      if (pupd) *reinterpret_cast<v2*>(p + i0) = ld_stream<v2>(reinterpret_cast<const v2*>(z + i0)) + beta * pv;
+      if (pupd) *reinterpret_cast<v2*>(p + i0) = ld_vec<!KEEP>(reinterpret_cast<const v2*>(z + i0)) + beta * pv;
       return;
     }
   }
@@ -387,7 +403,7 @@ __global__ __launch_bounds__(256) void cg_xpupdate_kernel(long long n, T* __rest
     if (i < n) {
       const T pv = p[i];
       st_stream<T>(ld_stream<T>(x + i) + lambda * pv, x + i);
-      if (pupd) p[i] = ld_stream<T>(z + i) + beta * pv;
+      if (pupd) p[i] = ld_vec<!KEEP>(z + i) + beta * pv;
     }
   }
 }

@@ -647,6 +647,7 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
   const bool fold_pq = !P.block() && nbapply <= kFoldPartials;
   const bool fold_check = n <= kFoldElements;  // and few enough of them
   const bool recompute = P.block() && !fold_check && bj_cg_recompute(h, P.trans);
+  const int cache = cg_cache(n * (long long)sizeof(T));
   const int rblocks = (int)std::min<long long>(kRedBlocks, (n + 2 * kRedThreads - 1) / (2 * kRedThreads));
   // point Jacobi: z = dinv r in b's place until the loop ends
   const T* zv = P.block() ? z : b;
@@ -676,8 +677,13 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
         hipLaunchKernelGGL(kernel, dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, b, (const T*)q, P.dinv, scal,
                            partial_buf<A>(h), (const int*)h->d_state, (const A*)dotp, (int)nbapply, rslot);
       };
-      if (fold_pq) run(cg_rupdate_kernel<T, A, true>);
-      else run(cg_rupdate_kernel<T, A, false>);
+      auto choose = [&](auto c) {
+        if (fold_pq) run(cg_rupdate_kernel<T, A, true, decltype(c)::value>);
+        else run(cg_rupdate_kernel<T, A, false, decltype(c)::value>);
+      };
+      if (cache == CG_ALL) choose(std::integral_constant<int, CG_ALL>{});
+      else if (cache == CG_KEEP) choose(std::integral_constant<int, CG_KEEP>{});
+      else choose(std::integral_constant<int, CG_STREAM>{});
     }
     if (fold_check && nparts <= kFoldPartials / 2) {
       hipLaunchKernelGGL((cg_xpcheck_kernel<T, A>), dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, x, p, zv,
@@ -691,8 +697,11 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
         CHK((bj_launch<T, A>(h, P.trans, BJ_CGX, v, nullptr)));
       } else {
         const dim3 grid((unsigned)((n + 256LL * xp_ept<T>() - 1) / (256LL * xp_ept<T>())));
-        hipLaunchKernelGGL((cg_xpupdate_kernel<T, A>), grid, dim3(256), 0, h->stream, n, x, p, zv, (const A*)scal,
-                           (const int*)h->d_state, i);
+        auto run = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, grid, dim3(256), 0, h->stream, n, x, p, zv, (const A*)scal, (const int*)h->d_state, i);
+        };
+        if (cache == CG_STREAM) run(cg_xpupdate_kernel<T, A, false>);
+        else run(cg_xpupdate_kernel<T, A, true>);
       }
     }
     HIPCHK(h, hipGetLastError());
