@@ -526,8 +526,10 @@ __global__ __launch_bounds__(64) void bicg_init_kernel(double* __restrict__ bs, 
 
 // p = r (first iteration) or p = r + beta (p - omega v); with POINT the preconditioned
 // direction y = dinv p in p's place: y = dinv r or y = dinv (r - beta omega v) + beta y. One
-// element per thread over an exact grid, as in cg_xpupdate_kernel.
-template <typename T, bool POINT>
+// element per thread over an exact grid, as in cg_xpupdate_kernel. DSTREAM, here and below: dinv
+// streams past the memory-side cache, for vectors that do not all fit there (cg_cache; 96^3 Q2 925 ->
+// 918, 64^3 Q3 559 -> 545 us per iteration; at 48^3 Q2, where they fit, 127 -> 131).
+template <typename T, bool POINT, bool DSTREAM>
 __global__ __launch_bounds__(256) void bicg_dir_kernel(long long n, T* __restrict__ p, const T* __restrict__ r,
                                                        const T* __restrict__ v, const T* __restrict__ dinv,
                                                        const double* __restrict__ bs, const int* __restrict__ state,
@@ -541,7 +543,7 @@ __global__ __launch_bounds__(256) void bicg_dir_kernel(long long n, T* __restric
   if (i0 + E <= n) {
     V pn = *reinterpret_cast<const V*>(r + i0);
     V d;
-    if constexpr (POINT) d = *reinterpret_cast<const V*>(dinv + i0);
+    if constexpr (POINT) d = ld_vec<DSTREAM>(reinterpret_cast<const V*>(dinv + i0));
     if (!first) {
       const V po = *reinterpret_cast<const V*>(p + i0), vo = ld_stream<V>(reinterpret_cast<const V*>(v + i0));
       if constexpr (POINT) pn = d * (pn - bo * vo) + beta * po;
@@ -570,7 +572,7 @@ __global__ __launch_bounds__(256) void prec_stop_kernel(long long n, const T* __
 }
 
 // First half step: r -= alpha v with the r.r partials; with POINT also y = dinv r
-template <typename T, typename A, bool POINT>
+template <typename T, typename A, bool POINT, bool DSTREAM>
 __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* __restrict__ r, const T* __restrict__ v,
                                                                 const T* __restrict__ dinv, T* __restrict__ y,
                                                                 const double* __restrict__ bs, A* __restrict__ partial,
@@ -588,7 +590,7 @@ __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* 
       if (i < n) {
         rv[u] = r[i];
         vv[u] = v[i];
-        if constexpr (POINT) dv[u] = dinv[i];
+        if constexpr (POINT) dv[u] = ld_vec<DSTREAM>(dinv + i);
       }
     }
 #pragma unroll

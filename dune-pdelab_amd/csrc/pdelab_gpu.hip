@@ -854,22 +854,24 @@ static int bicg_first_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool fi
   const int* st = h->d_state;
   const T *r = w.r, *v = w.v;
   const bool point = P.dinv != nullptr;
-  if (point)
-    hipLaunchKernelGGL((bicg_dir_kernel<T, true>), grid, dim3(256), 0, h->stream, n, w.p, r, v, P.dinv, bs, st, first);
-  else
-    hipLaunchKernelGGL((bicg_dir_kernel<T, false>), grid, dim3(256), 0, h->stream, n, w.p, r, v, P.dinv, bs, st, first);
+  const bool dstream = cg_cache(n * (long long)sizeof(T)) != CG_ALL;
+  auto dir = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, h->stream, n, w.p, r, v, P.dinv, bs, st, first); };
+  if (point && dstream) dir(bicg_dir_kernel<T, true, true>);
+  else if (point) dir(bicg_dir_kernel<T, true, false>);
+  else dir(bicg_dir_kernel<T, false, false>);
   if (P.launched()) CHK((bicg_prec<T, A>(h, P, w.p, w.y1)));
   const A* parts;
   int np;
   CHK((apply_dots<T, A, 1>(h, w.y1, w.v, P.trans, w.rt, &parts, &np)));
   bicg_scalar<A, 0>(h, parts, np, 2 * i - 1);
   A* part = partial_buf<A>(h);
-  if (point)
-    hipLaunchKernelGGL((bicg_half_kernel<T, A, true>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, w.r, v, P.dinv,
-                       w.y2, bs, part, st);
-  else
-    hipLaunchKernelGGL((bicg_half_kernel<T, A, false>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, w.r, v,
-                       P.dinv, (T*)nullptr, bs, part, st);
+  auto half = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, w.r, v, P.dinv,
+                       point ? w.y2 : (T*)nullptr, bs, part, st);
+  };
+  if (point && dstream) half(bicg_half_kernel<T, A, true, true>);
+  else if (point) half(bicg_half_kernel<T, A, true, false>);
+  else half(bicg_half_kernel<T, A, false, false>);
   bicg_scalar<A, 1>(h, part, kRedBlocks, 2 * i - 1);
   HIPCHK(h, hipGetLastError());
   return PDELAB_OK;
