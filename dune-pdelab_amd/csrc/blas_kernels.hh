@@ -528,7 +528,7 @@ __global__ __launch_bounds__(64) void bicg_init_kernel(double* __restrict__ bs, 
 // direction y = dinv p in p's place: y = dinv r or y = dinv (r - beta omega v) + beta y. One
 // element per thread over an exact grid, as in cg_xpupdate_kernel. DSTREAM, here and below: dinv
 // streams past the memory-side cache, for vectors that do not all fit there (cg_cache; 96^3 Q2 925 ->
-// 918, 64^3 Q3 559 -> 545 us per iteration; at 48^3 Q2, where they fit, 127 -> 131).
+// 918, 64^3 Q3 559 -> 545 us per iteration; at 48^3 Q2, where they fit, no gain: 127 and 131 us).
 template <typename T, bool POINT, bool DSTREAM>
 __global__ __launch_bounds__(256) void bicg_dir_kernel(long long n, T* __restrict__ p, const T* __restrict__ r,
                                                        const T* __restrict__ v, const T* __restrict__ dinv,

@@ -72,6 +72,7 @@ struct pdelab_gpu_gridoperator {
   bool diag_valid = false;
   double* w64[8] = {nullptr};
   float* w32[8] = {nullptr};
+  void *d_small = nullptr, *h_small = nullptr;  // hold the partials, scalars and states below
   double* d_part64 = nullptr;
   float* d_part32 = nullptr;
   double* d_scal64 = nullptr;

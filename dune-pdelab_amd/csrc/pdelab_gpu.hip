@@ -797,7 +797,6 @@ static int bicg_vecs(H* h, const Prec<T>& P, int base, T* x, T* r, BicgVecs<T>& 
     if (!s[7]) HIPCHK(h, hipMalloc(&s[7], sizeof(T) * h->N));
     w.y1 = s[7];
   } else if (!P.dinv) w.y2 = r;
-  if (!h->d_bscal) HIPCHK(h, hipMalloc(&h->d_bscal, sizeof(double) * 8));
   return ensure_applydot(h);
 }
 
@@ -1467,19 +1466,26 @@ int pdelab_gpu_create(const pdelab_config* cfg, const double* kappa_host, pdelab
     pdelab_gpu_destroy(h);
     return code;
   }
-  if (hipMalloc(&h->d_part64, sizeof(double) * kRedBlocks * 4) != hipSuccess) return bail("hipMalloc failed");
-  if (hipMalloc(&h->d_part32, sizeof(float) * kRedBlocks * 4) != hipSuccess) return bail("hipMalloc failed");
-  if (hipMalloc(&h->d_scal64, sizeof(double) * 16) != hipSuccess) return bail("hipMalloc failed");
-  if (hipMalloc(&h->d_scal32, sizeof(float) * 16) != hipSuccess) return bail("hipMalloc failed");
-  if (hipHostMalloc(&h->h_scal64, sizeof(double) * 16) != hipSuccess) return bail("hipHostMalloc failed");
-  if (hipHostMalloc(&h->h_scal32, sizeof(float) * 16) != hipSuccess) return bail("hipHostMalloc failed");
+  // partials, scalars and state of the loops: one allocation on either side
+  constexpr size_t kPart = kRedBlocks * 4;
+  if (hipMalloc(&h->d_small, sizeof(double) * (kPart + 16 + 8 + 4) + sizeof(float) * (kPart + 16) + sizeof(int) * 4) != hipSuccess)
+    return bail("hipMalloc failed");
+  h->d_part64 = static_cast<double*>(h->d_small);
+  h->d_scal64 = h->d_part64 + kPart;
+  h->d_bscal = h->d_scal64 + 16;
+  h->d_dstate = h->d_bscal + 8;
+  h->d_part32 = reinterpret_cast<float*>(h->d_dstate + 4);
+  h->d_scal32 = h->d_part32 + kPart;
+  h->d_state = reinterpret_cast<int*>(h->d_scal32 + 16);
+  if (hipHostMalloc(&h->h_small, sizeof(double) * (16 + 4) + sizeof(float) * 16 + sizeof(int) * 8) != hipSuccess)
+    return bail("hipHostMalloc failed");
+  h->h_scal64 = static_cast<double*>(h->h_small);
+  h->h_dstate = h->h_scal64 + 16;
+  h->h_scal32 = reinterpret_cast<float*>(h->h_dstate + 4);
+  h->h_state = reinterpret_cast<int*>(h->h_scal32 + 16);
   if (hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess) return bail("hipEventCreate failed");
   for (hipEvent_t& e : h->evk)
     if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return bail("hipEventCreate failed");
-  if (hipMalloc(&h->d_state, sizeof(int) * 4) != hipSuccess) return bail("hipMalloc failed");
-  if (hipMalloc(&h->d_dstate, sizeof(double) * 4) != hipSuccess) return bail("hipMalloc failed");
-  if (hipHostMalloc(&h->h_state, sizeof(int) * 8) != hipSuccess) return bail("hipHostMalloc failed");
-  if (hipHostMalloc(&h->h_dstate, sizeof(double) * 4) != hipSuccess) return bail("hipHostMalloc failed");
   if (init_scratch(h) != PDELAB_OK) return bail(h->err);
   if (cfg->kappa_per_cell) {
     if (!kappa_host) { g_create_error = "kappa_per_cell requires a kappa array"; pdelab_gpu_destroy(h); return PDELAB_ERR_INVALID_ARG; }
@@ -1497,8 +1503,7 @@ int pdelab_gpu_destroy(pdelab_gpu_gridoperator* h) {
   if (!h) return PDELAB_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   void* ptrs[] = {h->d_kappa, h->d_kappa32, h->d_R0, h->d_src, h->d_ftab, h->d_gtab, h->d_diag, h->d_dinv,
-                  h->d_dinv32, h->d_part64, h->d_part32, h->d_scal64, h->d_scal32, h->d_applydot,
-                  h->d_state, h->d_dstate, h->d_bscal, h->d_tab, h->d_fc64, h->d_fc32};
+                  h->d_dinv32, h->d_small, h->d_applydot, h->d_tab, h->d_fc64, h->d_fc32};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (double* p : h->os)
@@ -1511,10 +1516,7 @@ int pdelab_gpu_destroy(pdelab_gpu_gridoperator* h) {
     if (h->w64[i]) (void)hipFree(h->w64[i]);
     if (h->w32[i]) (void)hipFree(h->w32[i]);
   }
-  if (h->h_scal64) (void)hipHostFree(h->h_scal64);
-  if (h->h_scal32) (void)hipHostFree(h->h_scal32);
-  if (h->h_state) (void)hipHostFree(h->h_state);
-  if (h->h_dstate) (void)hipHostFree(h->h_dstate);
+  if (h->h_small) (void)hipHostFree(h->h_small);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   for (hipEvent_t e : h->evk)
     if (e) (void)hipEventDestroy(e);
