@@ -486,8 +486,10 @@ __global__ __launch_bounds__(256) void cg_pupdate_kernel(long long n, T* __restr
 // point Jacobi works inside the updates, p is kept only for a preconditioner with a launch of
 // its own, x is updated once and the FP64 matrix-core apply takes the dots: 24 vectors read or
 // written per iteration where one kernel per statement moved 31 (96^3 Q2 convection, 191 MB per
-// vector: 1130 -> 920 us per iteration; the updates run at 5.8 to 6.3 TB/s). Single-workgroup
-// kernels keep the solver's scalars in FP64:
+// vector: 1130 -> 920 us per iteration; the updates run at 5.8 to 6.3 TB/s). alpha and omega are
+// formed by every workgroup of the update that uses them, from up to kFoldPartials partials (two
+// launches fewer: 48^3 Q2 131 -> 121 us per iteration, 64^3 Q3 546 -> 538). Single-workgroup kernels
+// form the others and keep the solver's scalars in FP64:
 //   bs = {rho, rho_new, alpha, omega, beta}; state = {stopped, abort code, half steps};
 //   dstate = {defect, def0, reduction}.
 // Once state[0] is set every later kernel that writes x, r or the scalars returns at once, but
@@ -571,18 +573,26 @@ __global__ __launch_bounds__(256) void prec_stop_kernel(long long n, const T* __
     y[i] = dinv ? dinv[i] * x[i] : x[i];
 }
 
-// First half step: r -= alpha v with the r.r partials; with POINT also y = dinv r
-template <typename T, typename A, bool POINT, bool DSTREAM>
+// alpha of the half step from h = rt.v; false: abort, |h| < EPSILON
+__device__ __forceinline__ bool bicg_alpha(double h, const double* __restrict__ bs, const double* __restrict__ dstate,
+                                           double& alpha) {
+  alpha = dstate[0] == 0.0 ? 0.0 : bs[kBsRhoNew] / h;
+  return !(fabs(h) < kBicgEps);
+}
+
+// First half step: r -= alpha v with the r.r partials; with POINT also y = dinv r. FOLD: alpha from
+// the nd partials of rt.v at dots, by every workgroup (bicg_scalar_kernel's phase 0), else from bs.
+template <typename T, typename A, bool POINT, bool DSTREAM, bool FOLD>
 __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* __restrict__ r, const T* __restrict__ v,
                                                                 const T* __restrict__ dinv, T* __restrict__ y,
-                                                                const double* __restrict__ bs, A* __restrict__ partial,
-                                                                const int* __restrict__ state) {
-  if (state[0]) return;
-  const T alpha = (T)bs[kBsAlpha];
+                                                                double* bs, A* __restrict__ partial, int* state,
+                                                                const double* __restrict__ dstate,
+                                                                const A* __restrict__ dots, int nd) {
+  if (*(volatile int*)state) return;  // an abort below may set it while other workgroups start
   A s[1] = {A(0)};
   constexpr long long S = (long long)kRedBlocks * kRedThreads;
-  for (long long i0 = (long long)blockIdx.x * kRedThreads + threadIdx.x; i0 < n; i0 += kVecUnroll * S) {
-    T rv[kVecUnroll], vv[kVecUnroll], dv[kVecUnroll];
+  T rv[kVecUnroll], vv[kVecUnroll], dv[kVecUnroll];
+  auto load = [&](long long i0) {
 #pragma unroll
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
@@ -593,6 +603,26 @@ __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* 
         if constexpr (POINT) dv[u] = ld_vec<DSTREAM>(dinv + i);
       }
     }
+  };
+  const long long first = (long long)blockIdx.x * kRedThreads + threadIdx.x;
+  load(first);  // on their way while alpha is formed
+  T alpha;
+  if constexpr (FOLD) {
+    A h[1];
+    double al;
+    group_partial_sum<A, 1>(dots, nd, h);
+    const bool go = bicg_alpha((double)h[0], bs, dstate, al);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      if (go) bs[kBsAlpha] = al;
+      else {
+        state[1] = BICG_H;
+        state[0] = 1;
+      }
+    }
+    if (!go) return;
+    alpha = (T)al;
+  } else alpha = (T)bs[kBsAlpha];
+  for (long long i0 = first; i0 < n;) {
 #pragma unroll
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
@@ -603,6 +633,8 @@ __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* 
         s[0] += (A)ri * (A)ri;
       }
     }
+    i0 += kVecUnroll * S;
+    if (i0 < n) load(i0);
   }
   block_sum<A, 1>(s);
   if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
@@ -610,24 +642,27 @@ __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* 
 
 // Second half step `half`: x += alpha y1 + omega y2, r -= omega t with the (r.r, rt.r)
 // partials; y2 null: r before its update (no preconditioner); y1 null: its part is in x already.
-// If the first half step stopped the loop, only x += alpha y1.
-template <typename T, typename A>
+// If the first half step stopped the loop, only x += alpha y1. FOLD: omega from the nd pairs of
+// partials of (r.t, t.t) at dots, by every workgroup (bicg_scalar_kernel's phase 2), else from bs.
+template <typename T, typename A, bool FOLD>
 __global__ __launch_bounds__(kRedThreads) void bicg_full_kernel(long long n, T* __restrict__ x, const T* __restrict__ y1,
                                                                 const T* __restrict__ y2, T* __restrict__ r,
                                                                 const T* __restrict__ t, const T* __restrict__ rt,
-                                                                const double* __restrict__ bs, A* __restrict__ partial,
-                                                                const int* __restrict__ state, int half) {
+                                                                double* bs, A* __restrict__ partial,
+                                                                const int* __restrict__ state, int half,
+                                                                const double* __restrict__ dstate,
+                                                                const A* __restrict__ dots, int nd) {
   const long long first = (long long)blockIdx.x * kRedThreads + threadIdx.x;
   constexpr long long S = (long long)kRedBlocks * kRedThreads;
-  const T alpha = (T)bs[kBsAlpha], omega = (T)bs[kBsOmega];
+  const T alpha = (T)bs[kBsAlpha];
   if (state[0]) {
     if (state[2] == half - 1 && y1)
       for (long long i = first; i < n; i += S) x[i] += alpha * y1[i];
     return;
   }
   A s[2] = {A(0), A(0)};
-  for (long long i0 = first; i0 < n; i0 += kVecUnroll * S) {
-    T xv[kVecUnroll], av[kVecUnroll], bv[kVecUnroll], rv[kVecUnroll], tv[kVecUnroll], sv[kVecUnroll];
+  T xv[kVecUnroll], av[kVecUnroll], bv[kVecUnroll], rv[kVecUnroll], tv[kVecUnroll], sv[kVecUnroll];
+  auto load = [&](long long i0) {
 #pragma unroll
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
@@ -641,6 +676,17 @@ __global__ __launch_bounds__(kRedThreads) void bicg_full_kernel(long long n, T* 
         sv[u] = ld_stream<T>(rt + i);
       }
     }
+  };
+  load(first);  // on their way while omega is formed
+  T omega;
+  if constexpr (FOLD) {
+    A d[2];
+    group_partial_sum<A, 2>(dots, nd, d);
+    const double om = dstate[0] == 0.0 ? 0.0 : (double)d[0] / (double)d[1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) bs[kBsOmega] = om;
+    omega = (T)om;
+  } else omega = (T)bs[kBsOmega];
+  for (long long i0 = first; i0 < n;) {
 #pragma unroll
     for (int u = 0; u < kVecUnroll; ++u) {
       const long long i = i0 + u * S;
@@ -654,6 +700,8 @@ __global__ __launch_bounds__(kRedThreads) void bicg_full_kernel(long long n, T* 
         s[1] += (A)sv[u] * (A)ri;
       }
     }
+    i0 += kVecUnroll * S;
+    if (i0 < n) load(i0);
   }
   block_sum<A, 2>(s);
   if (threadIdx.x == 0) {
@@ -680,13 +728,13 @@ __global__ __launch_bounds__(kFinalThreads) void bicg_scalar_kernel(const A* __r
   if (threadIdx.x != 0) return;
   const double norm = dstate[0];
   if constexpr (PHASE == 0) {
-    const double hh = (double)v[0];
-    if (fabs(hh) < kBicgEps) {
+    double alpha;
+    if (!bicg_alpha((double)v[0], bs, dstate, alpha)) {
       state[1] = BICG_H;
       state[0] = 1;
       return;
     }
-    bs[kBsAlpha] = norm == 0.0 ? 0.0 : bs[kBsRhoNew] / hh;
+    bs[kBsAlpha] = alpha;
   } else if constexpr (PHASE == 1) {
     bicg_step(state, dstate, half, sqrt((double)v[0]));
   } else if constexpr (PHASE == 2) {

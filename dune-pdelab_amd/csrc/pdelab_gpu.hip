@@ -844,6 +844,10 @@ static void bicg_scalar(H* h, const A* parts, int nparts, int half) {
                      h->d_bscal, h->d_state, h->d_dstate, half);
 }
 
+// Partials of the updates' own sums, apart from those that apply_dots leaves and the updates read
+template <typename A>
+static A* bicg_part(H* h) { return partial_buf<A>(h) + 2 * kRedBlocks; }
+
 // First half step of iteration i: p, y1 = W^{-1} p, v = J y1, alpha, r -= alpha v
 template <typename T, typename A>
 static int bicg_first_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool first, int i) {
@@ -862,15 +866,16 @@ static int bicg_first_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool fi
   const A* parts;
   int np;
   CHK((apply_dots<T, A, 1>(h, w.y1, w.v, P.trans, w.rt, &parts, &np)));
-  bicg_scalar<A, 0>(h, parts, np, 2 * i - 1);
-  A* part = partial_buf<A>(h);
+  const bool fold = np <= kFoldPartials;
+  if (!fold) bicg_scalar<A, 0>(h, parts, np, 2 * i - 1);
+  A* part = bicg_part<A>(h);
   auto half = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, w.r, v, P.dinv,
-                       point ? w.y2 : (T*)nullptr, bs, part, st);
+                       point ? w.y2 : (T*)nullptr, h->d_bscal, part, h->d_state, (const double*)h->d_dstate, parts, np);
   };
-  if (point && dstream) half(bicg_half_kernel<T, A, true, true>);
-  else if (point) half(bicg_half_kernel<T, A, true, false>);
-  else half(bicg_half_kernel<T, A, false, false>);
+  if (point && dstream) fold ? half(bicg_half_kernel<T, A, true, true, true>) : half(bicg_half_kernel<T, A, true, true, false>);
+  else if (point) fold ? half(bicg_half_kernel<T, A, true, false, true>) : half(bicg_half_kernel<T, A, true, false, false>);
+  else fold ? half(bicg_half_kernel<T, A, false, false, true>) : half(bicg_half_kernel<T, A, false, false, false>);
   bicg_scalar<A, 1>(h, part, kRedBlocks, 2 * i - 1);
   HIPCHK(h, hipGetLastError());
   return PDELAB_OK;
@@ -884,11 +889,16 @@ static int bicg_second_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool r
   const A* parts;
   int np;
   CHK((apply_dots<T, A, 2>(h, w.y2, w.t, P.trans, w.r, &parts, &np)));
-  bicg_scalar<A, 2>(h, parts, np, 2 * i);
-  A* part = partial_buf<A>(h);
-  hipLaunchKernelGGL((bicg_full_kernel<T, A>), dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, h->N, w.x,
-                     resumed ? (const T*)nullptr : (const T*)w.y1, w.y2 == w.r ? (const T*)nullptr : (const T*)w.y2, w.r,
-                     (const T*)w.t, (const T*)w.rt, (const double*)h->d_bscal, part, (const int*)h->d_state, 2 * i);
+  const bool fold = np <= kFoldPartials;
+  if (!fold) bicg_scalar<A, 2>(h, parts, np, 2 * i);
+  A* part = bicg_part<A>(h);
+  auto full = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, h->N, w.x,
+                       resumed ? (const T*)nullptr : (const T*)w.y1, w.y2 == w.r ? (const T*)nullptr : (const T*)w.y2, w.r,
+                       (const T*)w.t, (const T*)w.rt, h->d_bscal, part, (const int*)h->d_state, 2 * i,
+                       (const double*)h->d_dstate, parts, np);
+  };
+  fold ? full(bicg_full_kernel<T, A, true>) : full(bicg_full_kernel<T, A, false>);
   bicg_scalar<A, 3>(h, part, kRedBlocks, 2 * i);
   HIPCHK(h, hipGetLastError());
   return PDELAB_OK;
@@ -896,9 +906,10 @@ static int bicg_second_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool r
 
 // BiCGSTABSolver::apply (dune-istl) with half-step iteration counting, as a device-side
 // loop: the scalars, the Iteration::step test and the breakdown checks run in
-// single-workgroup kernels (bicg_scalar_kernel), so an iteration enqueues its launches (9 on the
-// matrix-core path with point Jacobi) without waiting; the host reads the stop flag every
-// kBicgCheckEvery iterations.
+// single-workgroup kernels (bicg_scalar_kernel) or, alpha and omega where their partials are
+// few, inside the updates, so an iteration enqueues its launches (7 on the matrix-core path
+// with point Jacobi) without waiting; the host reads the stop flag every kBicgCheckEvery
+// iterations.
 template <typename T, typename A>
 static int bicgstab_solve(H* h, T* x, T* r, double reduction, int maxit, int precond, bool trans, int base,
                           pdelab_linear_solver_result* res) {
