@@ -490,7 +490,7 @@ __global__ __launch_bounds__(256) void cg_pupdate_kernel(long long n, T* __restr
 // formed by every workgroup of the update that uses them, from up to kFoldPartials partials (two
 // launches fewer: 48^3 Q2 131 -> 121 us per iteration, 64^3 Q3 546 -> 538). Single-workgroup kernels
 // form the others and keep the solver's scalars in FP64:
-//   bs = {rho, rho_new, alpha, omega, beta}; state = {stopped, abort code, half steps};
+//   bs = {rho, rho_new, alpha, omega, beta}; state = {not 0 once stopped, abort code, half steps};
 //   dstate = {defect, def0, reduction}.
 // Once state[0] is set every later kernel that writes x, r or the scalars returns at once, but
 // for the alpha part of x when it was the half step that stopped the loop: x and r are those of
@@ -580,15 +580,19 @@ __device__ __forceinline__ bool bicg_alpha(double h, const double* __restrict__ 
   return !(fabs(h) < kBicgEps);
 }
 
-// First half step: r -= alpha v with the r.r partials; with POINT also y = dinv r. FOLD: alpha from
-// the nd partials of rt.v at dots, by every workgroup (bicg_scalar_kernel's phase 0), else from bs.
+// First half step `half`: r -= alpha v with the r.r partials; with POINT also y = dinv r. FOLD: alpha
+// from the nd partials of rt.v at dots, by every workgroup (bicg_scalar_kernel's phase 0), else from
+// bs. On an abort workgroup 0 raises the flag as -half, which no wave of this launch obeys: a workgroup
+// that starts late may read it in some waves and not in others, and all of them have to meet at
+// the barrier of the sum, whose result sends every one of them away.
 template <typename T, typename A, bool POINT, bool DSTREAM, bool FOLD>
 __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* __restrict__ r, const T* __restrict__ v,
                                                                 const T* __restrict__ dinv, T* __restrict__ y,
                                                                 double* bs, A* __restrict__ partial, int* state,
-                                                                const double* __restrict__ dstate,
+                                                                int half, const double* __restrict__ dstate,
                                                                 const A* __restrict__ dots, int nd) {
-  if (*(volatile int*)state) return;  // an abort below may set it while other workgroups start
+  const int stopped = *(volatile int*)state;
+  if (stopped && stopped != -half) return;
   A s[1] = {A(0)};
   constexpr long long S = (long long)kRedBlocks * kRedThreads;
   T rv[kVecUnroll], vv[kVecUnroll], dv[kVecUnroll];
@@ -616,7 +620,7 @@ __global__ __launch_bounds__(kRedThreads) void bicg_half_kernel(long long n, T* 
       if (go) bs[kBsAlpha] = al;
       else {
         state[1] = BICG_H;
-        state[0] = 1;
+        state[0] = -half;
       }
     }
     if (!go) return;

@@ -871,7 +871,8 @@ static int bicg_first_half(H* h, const Prec<T>& P, const BicgVecs<T>& w, bool fi
   A* part = bicg_part<A>(h);
   auto half = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(kRedBlocks), dim3(kRedThreads), 0, h->stream, n, w.r, v, P.dinv,
-                       point ? w.y2 : (T*)nullptr, h->d_bscal, part, h->d_state, (const double*)h->d_dstate, parts, np);
+                       point ? w.y2 : (T*)nullptr, h->d_bscal, part, h->d_state, 2 * i - 1, (const double*)h->d_dstate,
+                       parts, np);
   };
   if (point && dstream) fold ? half(bicg_half_kernel<T, A, true, true, true>) : half(bicg_half_kernel<T, A, true, true, false>);
   else if (point) fold ? half(bicg_half_kernel<T, A, true, false, true>) : half(bicg_half_kernel<T, A, true, false, false>);
