@@ -342,8 +342,6 @@ template <typename T>
 static int apply_mode(H* h, const T* z, T* y, bool trans, int mode, T* dotp = nullptr,
                       const int* stop = nullptr) {
   CHK(check_outflow(h));
-  if (h->varb && mode == 2)
-    return fail(h, PDELAB_ERR_UNSUPPORTED, "velocity field: CG (non-symmetric operator), use BiCGSTAB");
   if constexpr (std::is_same<T, double>::value) {
     if (h->varb && mfma_vel_kernel(h)) return launch_apply_mfma_vel(h, z, y, trans, mode == 1, stop);
     if (mfma_kernel(h)) {
@@ -631,6 +629,8 @@ struct CgLoopOut {
 template <typename T, typename A>
 static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool trans, int maxit, double def_ref,
                    double red, CgLoopOut& out) {
+  if (h->varb)
+    return fail(h, PDELAB_ERR_UNSUPPORTED, "velocity field: CG (non-symmetric operator), use BiCGSTAB");
   const long long n = h->N;
   const long long nbapply = apply_partials<T>(h);
   CHK(ensure_applydot(h));
@@ -655,71 +655,76 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
     hipLaunchKernelGGL((cg_scale_kernel<T, false>), dim3(grid_for(n)), dim3(256), 0, h->stream, n, b, P.dinv);
   bool stopped = false;
   int last = 0;
-  for (int i = 1; i <= maxit && !stopped; ++i) {
-    const int rslot = (i & 1) ? 7 : 5;  // slot holding the current rho
-    const int oslot = (i & 1) ? 4 : 6;  // (def^2, rho_new) written here
-    // q = J p with the p.q partials -> scal[0]; r -= lambda q (as z) with the (r.r, z.r)
-    // partials -> scal[oslot..] and the defect check; x += lambda p, p = z + beta p
-    CHK(apply_mode<T>(h, p, q, trans, 2, dotp, h->d_state));
-    if (!fold_pq)
-      hipLaunchKernelGGL((cg_pq_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, (const A*)dotp, (int)nbapply,
-                         scal, rslot, (const int*)h->d_state);
-    const A* parts = partial_buf<A>(h);
-    int nparts = rblocks;
-    if (P.block()) {
-      // r -= lambda q and z = W^{-1} r in one pass over the cells (z is kept for the p update,
-      // or formed again there)
-      const BJVec<T, A> v{b, z, b, q, scal + kSlotLambda, nullptr, h->d_state};
-      CHK((bj_launch<T, A>(h, P.trans, recompute ? BJ_CGD : BJ_CGR, v, &nparts)));
-      parts = static_cast<const A*>(h->d_bjpart);
-    } else {
-      auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, b, (const T*)q, P.dinv, scal,
-                           partial_buf<A>(h), (const int*)h->d_state, (const A*)dotp, (int)nbapply, rslot);
-      };
-      auto choose = [&](auto c) {
-        if (fold_pq) run(cg_rupdate_kernel<T, A, true, decltype(c)::value>);
-        else run(cg_rupdate_kernel<T, A, false, decltype(c)::value>);
-      };
-      if (cache == CG_ALL) choose(std::integral_constant<int, CG_ALL>{});
-      else if (cache == CG_KEEP) choose(std::integral_constant<int, CG_KEEP>{});
-      else choose(std::integral_constant<int, CG_STREAM>{});
-    }
-    if (fold_check && nparts <= kFoldPartials / 2) {
-      hipLaunchKernelGGL((cg_xpcheck_kernel<T, A>), dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, x, p, zv,
-                         (const A*)scal, h->d_state, h->d_dstate, i, parts, nparts, (const A*)(scal + rslot),
-                         scal + oslot);
-    } else {
-      hipLaunchKernelGGL((cg_check_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, parts, nparts, scal + oslot,
-                         h->d_state, h->d_dstate, i, (const A*)(scal + rslot), scal + kSlotBeta);
-      if (recompute) {
-        const BJVec<T, A> v{b, nullptr, nullptr, nullptr, scal + kSlotLambda, nullptr, h->d_state, x, p, scal + kSlotBeta, i};
-        CHK((bj_launch<T, A>(h, P.trans, BJ_CGX, v, nullptr)));
+  auto iterate = [&]() -> int {
+    for (int i = 1; i <= maxit && !stopped; ++i) {
+      const int rslot = (i & 1) ? 7 : 5;  // slot holding the current rho
+      const int oslot = (i & 1) ? 4 : 6;  // (def^2, rho_new) written here
+      // q = J p with the p.q partials -> scal[0]; r -= lambda q (as z) with the (r.r, z.r)
+      // partials -> scal[oslot..] and the defect check; x += lambda p, p = z + beta p
+      CHK(apply_mode<T>(h, p, q, trans, 2, dotp, h->d_state));
+      if (!fold_pq)
+        hipLaunchKernelGGL((cg_pq_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, (const A*)dotp, (int)nbapply,
+                           scal, rslot, (const int*)h->d_state);
+      const A* parts = partial_buf<A>(h);
+      int nparts = rblocks;
+      if (P.block()) {
+        // r -= lambda q and z = W^{-1} r in one pass over the cells (z is kept for the p update,
+        // or formed again there)
+        const BJVec<T, A> v{b, z, b, q, scal + kSlotLambda, nullptr, h->d_state};
+        CHK((bj_launch<T, A>(h, P.trans, recompute ? BJ_CGD : BJ_CGR, v, &nparts)));
+        parts = static_cast<const A*>(h->d_bjpart);
       } else {
-        const dim3 grid((unsigned)((n + 256LL * xp_ept<T>() - 1) / (256LL * xp_ept<T>())));
         auto run = [&](auto kernel) {
-          hipLaunchKernelGGL(kernel, grid, dim3(256), 0, h->stream, n, x, p, zv, (const A*)scal, (const int*)h->d_state, i);
+          hipLaunchKernelGGL(kernel, dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, b, (const T*)q, P.dinv, scal,
+                             partial_buf<A>(h), (const int*)h->d_state, (const A*)dotp, (int)nbapply, rslot);
         };
-        if (cache == CG_STREAM) run(cg_xpupdate_kernel<T, A, false>);
-        else run(cg_xpupdate_kernel<T, A, true>);
+        auto choose = [&](auto c) {
+          if (fold_pq) run(cg_rupdate_kernel<T, A, true, decltype(c)::value>);
+          else run(cg_rupdate_kernel<T, A, false, decltype(c)::value>);
+        };
+        if (cache == CG_ALL) choose(std::integral_constant<int, CG_ALL>{});
+        else if (cache == CG_KEEP) choose(std::integral_constant<int, CG_KEEP>{});
+        else choose(std::integral_constant<int, CG_STREAM>{});
+      }
+      if (fold_check && nparts <= kFoldPartials / 2) {
+        hipLaunchKernelGGL((cg_xpcheck_kernel<T, A>), dim3(rblocks), dim3(kRedThreads), 0, h->stream, n, x, p, zv,
+                           (const A*)scal, h->d_state, h->d_dstate, i, parts, nparts, (const A*)(scal + rslot),
+                           scal + oslot);
+      } else {
+        hipLaunchKernelGGL((cg_check_kernel<A>), dim3(1), dim3(kFinalThreads), 0, h->stream, parts, nparts, scal + oslot,
+                           h->d_state, h->d_dstate, i, (const A*)(scal + rslot), scal + kSlotBeta);
+        if (recompute) {
+          const BJVec<T, A> v{b, nullptr, nullptr, nullptr, scal + kSlotLambda, nullptr, h->d_state, x, p, scal + kSlotBeta, i};
+          CHK((bj_launch<T, A>(h, P.trans, BJ_CGX, v, nullptr)));
+        } else {
+          const dim3 grid((unsigned)((n + 256LL * xp_ept<T>() - 1) / (256LL * xp_ept<T>())));
+          auto run = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, h->stream, n, x, p, zv, (const A*)scal, (const int*)h->d_state, i);
+          };
+          if (cache == CG_STREAM) run(cg_xpupdate_kernel<T, A, false>);
+          else run(cg_xpupdate_kernel<T, A, true>);
+        }
+      }
+      HIPCHK(h, hipGetLastError());
+      last = i;
+      // The flag is read while the next kCheckEvery iterations run: the stream never drains. What
+      // was enqueued after the stop returns at once.
+      if (i % kCheckEvery == 0 || i == maxit) {
+        const int k = i / kCheckEvery & 1;
+        HIPCHK(h, hipMemcpyAsync(h->h_state + 4 * k, h->d_state, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipEventRecord(h->evk[k], h->stream));
+        if (i > kCheckEvery) {
+          HIPCHK(h, hipEventSynchronize(h->evk[k ^ 1]));
+          stopped = h->h_state[4 * (k ^ 1)] != 0;
+        }
       }
     }
-    HIPCHK(h, hipGetLastError());
-    last = i;
-    // The flag is read while the next kCheckEvery iterations run: the stream never drains. What
-    // was enqueued after the stop returns at once.
-    if (i % kCheckEvery == 0 || i == maxit) {
-      const int k = i / kCheckEvery & 1;
-      HIPCHK(h, hipMemcpyAsync(h->h_state + 4 * k, h->d_state, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
-      HIPCHK(h, hipEventRecord(h->evk[k], h->stream));
-      if (i > kCheckEvery) {
-        HIPCHK(h, hipEventSynchronize(h->evk[k ^ 1]));
-        stopped = h->h_state[4 * (k ^ 1)] != 0;
-      }
-    }
-  }
+    return PDELAB_OK;
+  };
+  const int status = iterate();
   if (P.dinv)
     hipLaunchKernelGGL((cg_scale_kernel<T, true>), dim3(grid_for(n)), dim3(256), 0, h->stream, n, b, P.dinv);
+  CHK(status);  // after b is r again
   HIPCHK(h, hipMemcpyAsync(h->h_state, h->d_state, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipMemcpyAsync(h->h_dstate, h->d_dstate, sizeof(double) * 4, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));

@@ -25,3 +25,23 @@ def test_bicgstab_abort_leaves_x_and_r(pkg, grid, degree):
             go.solve(xd, rd, method=pkg.SOLVER_BICGSTAB, precond=0, reduction=1e-10, maxit=3)
         assert np.array_equal(rd.download(), b)
         assert not xd.download().any()
+
+
+@pytest.mark.parametrize("precond", [0, 1, 2], ids=["none", "point", "block"])
+def test_refused_cg_leaves_the_defect(pkg, precond):
+    """CG is refused with a velocity field: x keeps its bits and r is the defect of x, in which
+    dune-istl's solvers take and leave it."""
+    print(f"[gpu] refused CG precond {precond}", flush=True)
+    cfg = pkg.make_config(nx=5, ny=4, nz=3, degree=2, alpha=3.0)
+    go = pkg.GridOperator(cfg)
+    rng = np.random.default_rng(32)
+    m = pkg.quadrature_points(cfg)
+    go.set_velocity_field(rng.normal(size=60 * 3 * m ** 3), rng.normal(size=(6 * 12 + 5 * 15 + 20 * 4) * m ** 2))
+    b, x0 = rng.uniform(-1, 1, go.N), rng.uniform(-1, 1, go.N)
+    xd, rd, jx = go.vector(x0), go.vector(b), go.vector()
+    go.operator_apply(xd, jx)
+    with pytest.raises(pkg.PdelabError, match="CG"):
+        go.solve(xd, rd, method=pkg.SOLVER_CG, precond=precond, reduction=1e-10, maxit=5)
+    assert np.array_equal(xd.download(), x0)
+    # one multiply-add per entry, fused or not: two roundings of |b| + |Jx|
+    assert np.all(np.abs(rd.download() - (b - jx.download())) <= 2.3e-16 * (np.abs(b) + np.abs(jx.download())))
