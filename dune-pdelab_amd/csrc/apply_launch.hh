@@ -18,33 +18,24 @@ static int launch_apply_walk(H* h, const T* z, T* y, const T* fc, const DGArgs<T
 template <int N1, typename T, bool TRANS, bool CONV, bool REACT, bool VARK, bool ACCUM, bool DOT>
 static int launch_apply_k(H* h, const T* z, T* y, const T* fc, const DGArgs<T>& a, T* dotp, const int* stop) {
   using SH = ApplyShape<N1>;
+  const long long nb = apply_blocks(h);
   const LineMats<T>* lm = line_mats<T>(h, TRANS);
-  if constexpr (sizeof(T) == 8 && N1 >= 3) {
-    // Q2 and Q3 in FP64 come here only where the matrix-core kernel does not apply
-    const long long nb = apply_blocks_of(h, false);
+  const int zw = apply_walk(h);
+  if constexpr (!VARK && !CONV && N1 == 4) {
+    if (zw == 2) return launch_apply_walk<N1, T, TRANS, REACT, ACCUM, DOT, 2>(h, z, y, fc, a, lm, nb, dotp, stop);
+  }
+  if constexpr (!VARK && !CONV && N1 == 3) {
+    if (zw == 8) return launch_apply_walk<N1, T, TRANS, REACT, ACCUM, DOT, 8>(h, z, y, fc, a, lm, nb, dotp, stop);
+    if (zw == 4) return launch_apply_walk<N1, T, TRANS, REACT, ACCUM, DOT, 4>(h, z, y, fc, a, lm, nb, dotp, stop);
+  }
+  if (row_kernel(h))
+    hipLaunchKernelGGL((dg_apply_rowreg_kernel<N1, T, TRANS, CONV, REACT, VARK, ACCUM, DOT>), dim3((unsigned)nb),
+                       dim3(SH::THREADS), 0, h->stream, z, y, fc, a, lm, nb, dotp, stop);
+  else
     hipLaunchKernelGGL((dg_apply_kernel<N1, T, TRANS, CONV, REACT, VARK, ACCUM, DOT>), dim3((unsigned)nb),
                        dim3(SH::THREADS), 0, h->stream, z, y, fc, a, lm, nb, dotp, stop);
-    HIPCHK(h, hipGetLastError());
-    return PDELAB_OK;
-  } else {
-    const long long nb = apply_blocks(h);
-    const int zw = apply_walk(h);
-    if constexpr (!VARK && !CONV && N1 == 4) {
-      if (zw == 2) return launch_apply_walk<N1, T, TRANS, REACT, ACCUM, DOT, 2>(h, z, y, fc, a, lm, nb, dotp, stop);
-    }
-    if constexpr (!VARK && !CONV && N1 == 3) {
-      if (zw == 8) return launch_apply_walk<N1, T, TRANS, REACT, ACCUM, DOT, 8>(h, z, y, fc, a, lm, nb, dotp, stop);
-      if (zw == 4) return launch_apply_walk<N1, T, TRANS, REACT, ACCUM, DOT, 4>(h, z, y, fc, a, lm, nb, dotp, stop);
-    }
-    if (row_kernel(h))
-      hipLaunchKernelGGL((dg_apply_rowreg_kernel<N1, T, TRANS, CONV, REACT, VARK, ACCUM, DOT>), dim3((unsigned)nb),
-                         dim3(SH::THREADS), 0, h->stream, z, y, fc, a, lm, nb, dotp, stop);
-    else
-      hipLaunchKernelGGL((dg_apply_kernel<N1, T, TRANS, CONV, REACT, VARK, ACCUM, DOT>), dim3((unsigned)nb),
-                         dim3(SH::THREADS), 0, h->stream, z, y, fc, a, lm, nb, dotp, stop);
-    HIPCHK(h, hipGetLastError());
-    return PDELAB_OK;
-  }
+  HIPCHK(h, hipGetLastError());
+  return PDELAB_OK;
 }
 
 template <int N1, typename T, bool TRANS, bool CONV, bool VARK, bool ACCUM, bool DOT>

@@ -1,35 +1,28 @@
 // apply_mfma.hip -- launches of the matrix-core apply (dg_mfma.hh): Q2 and Q3 in FP64.
 #include "handle.hh"
 
-template <int N1, int KIND>
-static void launch_mode(H* h, const double* z, double* y, const MfmaTab* tab, const MfmaArgs& a, unsigned nb, int mode,
-                        double* dotp, const int* stop, const double* w) {
-  const double* fc = KIND == MFMA_WEIGHT || KIND == MFMA_TENSOR ? h->d_fw64 : h->d_fc64;
-  auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, h->stream, z, y, fc, tab, a, nb, dotp, stop, w);
-  };
+// f(kernel) with the instance of a degree, coefficient form and mode
+template <int N1, int KIND, typename F>
+static void with_mode(int mode, F f) {
   switch (mode) {
-    case 1: run(dg_mfma_kernel<N1, KIND, 1>); break;
-    case 2: run(dg_mfma_kernel<N1, KIND, 2>); break;
-    case 3: run(dg_mfma_kernel<N1, KIND, 3>); break;
-    case 4: run(dg_mfma_kernel<N1, KIND, 4>); break;
-    case 5: run(dg_mfma_kernel<N1, KIND, 5>); break;
-    default: run(dg_mfma_kernel<N1, KIND, 0>); break;
+    case 1: f(dg_mfma_kernel<N1, KIND, 1>); break;
+    case 2: f(dg_mfma_kernel<N1, KIND, 2>); break;
+    case 3: f(dg_mfma_kernel<N1, KIND, 3>); break;
+    case 4: f(dg_mfma_kernel<N1, KIND, 4>); break;
+    case 5: f(dg_mfma_kernel<N1, KIND, 5>); break;
+    default: f(dg_mfma_kernel<N1, KIND, 0>); break;
   }
 }
-
-template <int N1>
-static void launch_kind(H* h, const double* z, double* y, const MfmaTab* tab, const MfmaArgs& a, unsigned nb, int mode,
-                        double* dotp, const int* stop, const double* w) {
-  if (!h->vark) {
-    if (h->sym[0] && h->sym[1]) launch_mode<N1, MFMA_CONST>(h, z, y, tab, a, nb, mode, dotp, stop, w);
-    else launch_mode<N1, MFMA_CONV>(h, z, y, tab, a, nb, mode, dotp, stop, w);
+template <int N1, typename F>
+static void with_kind(int kind, int mode, F f) {
+  switch (kind) {
+    case MFMA_CONST: with_mode<N1, MFMA_CONST>(mode, f); break;
+    case MFMA_CONV: with_mode<N1, MFMA_CONV>(mode, f); break;
+    case MFMA_GENERAL: with_mode<N1, MFMA_GENERAL>(mode, f); break;
+    case MFMA_TENSOR: with_mode<N1, MFMA_TENSOR>(mode, f); break;
+    default: with_mode<N1, MFMA_WEIGHT>(mode, f); break;
   }
-  else if (h->conv || !h->a64.weightsOn) launch_mode<N1, MFMA_GENERAL>(h, z, y, tab, a, nb, mode, dotp, stop, w);
-  else if (h->a64.aniso) launch_mode<N1, MFMA_TENSOR>(h, z, y, tab, a, nb, mode, dotp, stop, w);
-  else launch_mode<N1, MFMA_WEIGHT>(h, z, y, tab, a, nb, mode, dotp, stop, w);
 }
-
 // Arguments of one launch without the field's.
 MfmaArgs mfma_args(const H* h, bool trans) {
   MfmaArgs a;
@@ -61,8 +54,13 @@ int launch_apply_mfma(H* h, const double* z, double* y, bool trans, int mode, do
   const unsigned nb = (unsigned)mfma_blocks(h);
   // J and J^T, each with the whole matrices and with their convection part (cell-wise kappa)
   const MfmaTab* tab = h->d_tab->mfma + (trans ? 1 : 0) + (h->vark ? 2 : 0);
-  if (h->n1 == 3) launch_kind<3>(h, z, y, tab, a, nb, mode, dotp, stop, w);
-  else launch_kind<4>(h, z, y, tab, a, nb, mode, dotp, stop, w);
+  const int kind = mfma_kind(h, false);
+  const double* fc = kind == MFMA_WEIGHT || kind == MFMA_TENSOR ? h->d_fw64 : h->d_fc64;
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, h->stream, z, y, fc, tab, a, nb, dotp, stop, w);
+  };
+  if (h->n1 == 3) with_kind<3>(kind, mode, run);
+  else with_kind<4>(kind, mode, run);
   HIPCHK(h, hipGetLastError());
   return PDELAB_OK;
 }

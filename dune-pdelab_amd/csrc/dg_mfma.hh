@@ -21,7 +21,7 @@
 // region of its own: no workgroup barrier, the next step's loads in flight during a step.
 // A boundary face replaces its cell's matrices, so cell-wise coefficients, convection,
 // transposition and partial rows (any nx: a block whose row ends ignores its neighbour)
-// take the same path. Q2 pads the 4x4 blocks with zeros.
+// take the same path. Q2 pads the 4x4 blocks with zeros. mfma_kernel() says which calls come here.
 //
 // Measured (y = J z, three states in turn, row kernel -> this one): 64^3 Q3 76.2 -> 61.6 us (268 MB,
 // 4.4 TB/s; reads 1.17x and writes 1.0x the algorithmic bytes; without memory traffic 31 us, so

@@ -147,12 +147,12 @@ inline long long apply_cpb(const H* h) {
   return h->n1 == 2 ? ApplyShape<2>::CPB : (h->n1 == 3 ? ApplyShape<3>::CPB : ApplyShape<4>::CPB);
 }
 
-// Whether an apply launch in FP32, or of Q1, takes the row kernel (chunks of x-rows) rather than
-// the general kernel (chunks of consecutive cells). Rows that split into whole chunks always do. The
-// partial last chunk of a row is moved back to overlap the previous one (nx > CPB), and
-// its overlapping lanes do work that is not stored, so such grids take the row kernel only
-// for the constant-coefficient symmetric operator, where it is fastest (0.78 of the
-// general kernel's time at Q3, 0.90 at Q2), with at most 1/8 (Q3) or 1/16 (Q2) of the
+// Whether an apply launch that the matrix cores do not take (FP32, Q1, see mfma_kernel) takes the
+// row kernel (chunks of x-rows) rather than the general kernel (chunks of consecutive cells). Rows
+// that split into whole chunks always do. The partial last chunk of a row is moved back to overlap
+// the previous one (nx > CPB), and its overlapping lanes do work that is not stored, so such grids
+// take the row kernel only for the constant-coefficient symmetric operator, where it is fastest
+// (0.78 of the general kernel's time at Q3, 0.90 at Q2), with at most 1/8 (Q3) or 1/16 (Q2) of the
 // row's lanes wasted. Decided per launch: set_kappa may change the operator after creation.
 inline bool row_kernel(const H* h) {
   if (h->apply_variant != 0) return false;
@@ -184,23 +184,65 @@ inline int apply_walk(const H* h) {
   return 1;
 }
 
-// Whether an FP64 apply takes the matrix-core kernel (dg_mfma.hh): Q2 and Q3, planes of at
-// least four cells (a wave's group) whose byte offsets stay below 4 GiB. It is faster than the
-// row and general kernels on every grid measured (row or general kernel -> this one, three
-// states in turn): 64^3 Q3 78.6 -> 61.6 us, convection 105.5 -> 66.3, lognormal kappa 117.5 ->
-// 71.7; 96^3 Q2 145.1 -> 116.6, 204.2 -> 128.9, 265.0 -> 160.2; 83x61x71 Q2 lognormal 116.8 ->
-// 65.6; 100^3 Q3 337.5 -> 258.7; 32^3 Q2 7.5 -> 5.0; 24^3 Q3 5.8 -> 4.5. A Q1 cell would fill an
-// eighth of the 4x4x4 blocks.
-inline bool mfma_kernel(const H* h) {
+// The coefficient form of a matrix-core launch (dg_mfma.hh)
+inline int mfma_kind(const H* h, bool vel) {
+  if (!h->vark) return vel || (h->sym[0] && h->sym[1]) ? MFMA_CONST : MFMA_CONV;
+  if (h->conv || !h->a64.weightsOn || (vel && h->a64.aniso)) return MFMA_GENERAL;
+  return h->a64.aniso ? MFMA_TENSOR : MFMA_WEIGHT;
+}
+
+// Whether the matrix-core kernel (dg_mfma.hh) can take an FP64 apply: Q2 and Q3, planes of at least
+// four cells (a wave's group) whose byte offsets stay below 4 GiB. A Q1 cell would fill an eighth of
+// the 4x4x4 blocks.
+inline bool mfma_shape(const H* h) {
   const long long np = (long long)h->a64.n[0] * h->a64.n[1];
   return h->apply_variant == 0 && h->n1 >= 3 && np >= 4 && np * h->nloc * 8 < (1LL << 32);
 }
+// Workgroups of a plane (16 cells each). Beyond about a thousand steps of workgroups along z a launch is
+// bound by its work, below by a wave's latency, where this kernel is always the faster one.
+inline long long mfma_wgs(const H* h) { return ((long long)h->a64.n[0] * h->a64.n[1] + 15) / 16; }
 
-// Whether its velocity-field form applies: up to four points per direction (Q2 with intorderadd
-// 0..3, Q3 with 0 or 1), the field's in-plane byte offsets below 4 GiB.
+// Whether it does. us, row or general kernel -> matrix cores: 64^3 Q3 78.6 -> 61.6, convection 105.5 ->
+// 66.3, lognormal kappa 117.5 -> 71.7; 96^3 Q2 145.1 -> 116.6, 204.2 -> 128.9, 265.0 -> 160.2; 83x61x71 Q2
+// lognormal 116.8 -> 65.6; 100^3 Q3 337.5 -> 258.7; 32^3 Q2 7.5 -> 5.0; 24^3 Q3 5.8 -> 4.5. The other two
+// kernels are the faster ones for
+// * cell-wise kappa with convection or weightsOff, whose lane matrices are combined from nine
+//   tables per face and step: 64^3 Q2 62 and 74 against 100, 96^3 Q3 445 and 463 against 604; small
+//   grids 7.8 -> 6.0 (8^3 Q2);
+// * planes that leave much of their last workgroup's 16 cells idle: 2x2x8192 Q2 9.5 against 19.3,
+//   17x1x8192 Q2 25.6 against 33.6. The share of busy cells at which that ends depends on the
+//   degree and the coefficient (Q2 constant 13 of 16, since there the others come closest);
+// * one plane of 128^2 cells or more, where each start serves a single step: 512x512x1 Q2 32 against 44 us
+//   (two planes 62 against 70), Q3 55 against 60; if rows split into whole chunks also with a diagonal
+//   tensor (57 against 66, J^T at Q3 105 against 125) and with cell-wise kappa at Q2 (56 against 60; at Q3
+//   y = J z 96 against 99, but J^T 110 against 102). Convection stays here (52 -> 44, Q3 95 -> 58).
+// fused: r += R(x), where the other kernels need a second pass over three vectors. That moves the lines:
+// 512x512x1 Q2 61 -> 54 us, 6x6x8192 Q2 77 -> 64; cell-wise kappa with convection 64^3 Q3 192 -> 166, 32^3 Q2
+// 21 -> 17 (48^3 Q2 52 against 55).
+inline bool mfma_kernel(const H* h, bool fused = false) {
+  if (!mfma_shape(h)) return false;
+  const int kind = mfma_kind(h, false);
+  const bool q2 = h->n1 == 3;
+  const long long wgs = mfma_wgs(h), np = (long long)h->a64.n[0] * h->a64.n[1], nz = h->a64.n[2], steps = wgs * nz;
+  if (kind == MFMA_GENERAL) return steps < (fused ? 2500 : 256) || (fused && !q2 && nz > 1 && np >= 13 * wgs);
+  const long long busy = kind == MFMA_CONV ? (q2 ? 8 : 6) : (q2 && kind == MFMA_CONST ? 13 : 9);
+  if (steps > 1024 && np < (fused ? std::min(busy, 7LL) : busy) * wgs) return false;
+  if (!fused && np >= 128 * 128 && nz <= (q2 && kind == MFMA_CONST ? 2 : 1)) {
+    if (kind == MFMA_CONST) return false;
+    if (kind == MFMA_TENSOR || (q2 && kind == MFMA_WEIGHT)) return !row_kernel(h);
+  }
+  return true;
+}
+
+// Whether its velocity-field form does: up to four points per direction (Q2 with intorderadd 0..3, Q3
+// with 0 or 1), the field's in-plane byte offsets below 4 GiB. It replaces two kernels and is the
+// slower one only on the thinnest planes: 2x2x8192 Q2 59 against 47 us, with a diagonal tensor or
+// weightsOff 91 against 50 (Q3 116 against 85; 4x2x8192 92 against 90).
 inline bool mfma_vel_kernel(const H* h) {
   const long long np = (long long)h->a64.n[0] * h->a64.n[1], m = h->tab.m;
-  return mfma_kernel(h) && m <= 4 && (h->vark || (h->sym[0] && h->sym[1])) && np * 6 * m * m * m * 8 < (1LL << 32);
+  if (!mfma_shape(h) || m > 4 || !(h->vark || (h->sym[0] && h->sym[1])) || np * 6 * m * m * m * 8 >= (1LL << 32)) return false;
+  const long long busy = mfma_kind(h, true) == MFMA_GENERAL ? 8 : (h->n1 == 3 ? 6 : 4);
+  return mfma_wgs(h) * h->a64.n[2] <= 1024 || np >= busy * mfma_wgs(h);
 }
 
 // One launch of the matrix-core apply: workgroups of four waves of four cells cover a plane,
@@ -214,9 +256,9 @@ struct MfmaGrid {
   int zsegs, zw;
 };
 inline MfmaGrid mfma_grid(const H* h) {
-  const long long np = (long long)h->a64.n[0] * h->a64.n[1], nz = h->a64.n[2];
+  const long long nz = h->a64.n[2];
   MfmaGrid g;
-  g.wgs = (np + 15) / 16;
+  g.wgs = mfma_wgs(h);
   auto cover = [&](long long target) { return (target + g.wgs - 1) / g.wgs; };
   const long long segs = std::max({(nz + 31) / 32, std::min(cover(1024), (nz + 7) / 8), std::min(cover(512), nz)});
   g.zw = (int)((nz + segs - 1) / segs);

@@ -373,7 +373,7 @@ static int apply_t(H* h, const T* z, T* y, bool trans, bool accum) {
 // kernel covers apply_walk(h) chunks)
 template <typename T>
 static long long apply_partials(H* h) {
-  if (sizeof(T) == 8 && h->n1 >= 3) return mfma_kernel(h) ? mfma_blocks(h) : apply_blocks_of(h, false);
+  if (sizeof(T) == 8 && mfma_kernel(h)) return mfma_blocks(h);
   return apply_blocks(h) / apply_walk(h);
 }
 
@@ -1652,7 +1652,7 @@ int pdelab_gpu_synchronize(pdelab_gpu_gridoperator* h) {
 int pdelab_gpu_residual(pdelab_gpu_gridoperator* h, const double* x, double* r) {
   if (!h || !x || !r) return PDELAB_ERR_INVALID_ARG;
   CHK(compute_R0(h));
-  if (!h->varb && mfma_kernel(h)) {  // R(0) inside the apply: a pass of its own took 73 us at 64^3 Q3
+  if (!h->varb && mfma_kernel(h, true)) {  // R(0) inside the apply: a pass of its own took 73 us at 64^3 Q3
     CHK(check_outflow(h));
     return launch_apply_mfma(h, x, r, false, 5, nullptr, nullptr, h->d_R0);
   }
