@@ -35,6 +35,8 @@ MfmaArgs mfma_args(const H* h, bool trans) {
   const MfmaGrid grid = mfma_grid(h);
   a.zw = grid.zw;
   a.zsegs = grid.zsegs;
+  a.prow = grid.prow;
+  a.prows = grid.prow ? (unsigned)(grid.wgs / grid.prow) : 0;
   a.vc = d.vc;
   for (int i = 0; i < 3; ++i) a.S[i] = d.S[i];
   a.fg = trans ? -d.theta : 1.0;

@@ -81,6 +81,7 @@ struct MfmaArgs {
   int nx, ny, nz;
   unsigned np;     // cells of a plane
   int zw, zsegs;   // z-steps of a wave, waves per column
+  unsigned prow, prows;  // workgroups of a row (rounded up) and such rows of a plane, if walked in strips; else 0
   double vc;       // reaction V c
   // cell-wise kappa: S per direction, face signs (1, theta) of J or (-theta, -1) of J^T,
   // Dirichlet penalty factor, boundary types
@@ -222,6 +223,21 @@ struct MfmaStage {
   }
 };
 
+// Position in the plane of workgroup w: in memory order, or (prow > 0) in strips of kMfmaStrip workgroups
+// along x, row after row. A row of workgroups is a row of cells rounded up, so that the strip drifts by
+// less than a workgroup per row where 16 does not divide nx; what is left of the plane follows in order.
+constexpr unsigned kMfmaStrip = 8;
+__host__ __device__ __forceinline__ unsigned mfma_strip(unsigned w, unsigned prow, unsigned prows) {
+  if (prow == 0 || w >= prow * prows) return w;
+  const unsigned full = prow / kMfmaStrip * kMfmaStrip;
+  if (w < full * prows) {
+    const unsigned s = w / (kMfmaStrip * prows), r = w % (kMfmaStrip * prows);
+    return r / kMfmaStrip * prow + s * kMfmaStrip + r % kMfmaStrip;
+  }
+  const unsigned r = w - full * prows, width = prow - full;
+  return r / width * prow + full + r % width;
+}
+
 // Orders a wave's LDS writes before its later reads (the LDS serves one wave's accesses in
 // order; this keeps the compiler from moving them).
 __device__ __forceinline__ void wave_lds_fence() {
@@ -283,7 +299,7 @@ __global__ __launch_bounds__(256, (VEL ? 2 : mfma_waves<N1, KIND, MODE>())) void
   const bool act = N1 == 4 || (i4 < N1 && k4 < N1);
   const unsigned lb = (unsigned)xcd_logical_block(blockIdx.x, nblocks);
   const unsigned gq = nblocks / (unsigned)a.zsegs, zs = lb / gq;
-  const unsigned c4 = 4u * (lb % gq * 4u + wave);  // first cell of the group
+  const unsigned c4 = 4u * (mfma_strip(lb % gq, a.prow, a.prows) * 4u + wave);  // first cell of the group
   const unsigned cs = min(c4, a.np - 4u);  // the last group is moved back to end with the plane
   const unsigned cc = cs + blk, nx = (unsigned)a.nx;
   const bool valid = cc >= c4;  // false for cells of the previous group (and past the plane): not stored

@@ -251,18 +251,25 @@ inline bool mfma_vel_kernel(const H* h) {
 // (four waves per SIMD), and shorter only for 512 workgroups. Walks of 4 / 8 / 16 / 32 steps:
 // 64^3 Q3 72 / 63 / 62 / 61 us, 64^3 Q2 - / 34.2 / 33.8 / 36.9 us; of 1 / 2 / 4: 32^3 Q2 7.5 / 7.0 /
 // 6.9 us.
+// Wide planes are walked in strips of 8 workgroups along x (mfma_strip): the 128 workgroups that an XCD
+// holds are 2048 consecutive cells, whose y-neighbours its L2 keeps only if that is many rows.
+// 2048x64x32 Q3 1693 -> 1034 us (row kernel 1240), 1024x32x32 Q3 362 -> 246 (row kernel 323), 512x128x32
+// Q3 681 -> 503 (624), 2048x64x32 Q2 719 -> 534, 384x128x32 Q3 412 -> 382; 256x256 gains 5 % at Q3 and loses
+// 1 % at 200x200; fewer than 8 planes lose up to 15 % at Q2.
 struct MfmaGrid {
   long long wgs;  // workgroups of a plane
   int zsegs, zw;
+  unsigned prow;  // workgroups of a row where the plane is walked in strips, else 0
 };
 inline MfmaGrid mfma_grid(const H* h) {
-  const long long nz = h->a64.n[2];
+  const long long nx = h->a64.n[0], nz = h->a64.n[2];
   MfmaGrid g;
   g.wgs = mfma_wgs(h);
   auto cover = [&](long long target) { return (target + g.wgs - 1) / g.wgs; };
   const long long segs = std::max({(nz + 31) / 32, std::min(cover(1024), (nz + 7) / 8), std::min(cover(512), nz)});
   g.zw = (int)((nz + segs - 1) / segs);
   g.zsegs = (int)((nz + g.zw - 1) / g.zw);
+  g.prow = nx > 256 && h->a64.n[1] > 1 && nz >= 8 ? (unsigned)((nx + 15) / 16) : 0u;
   return g;
 }
 inline long long mfma_blocks(const H* h) {

@@ -23,13 +23,16 @@ KINDS = {
 }
 # cell-wise kappa with convection or weightsOff: 255, 256 and more steps of workgroups, with whole and
 # partial chunks of the row kernel; thin planes of 4, 5, 17 and 18 cells past 1024 steps; one and
-# two planes of 128^2 cells, whole and partial chunks
+# two planes of 128^2 cells, whole and partial chunks; wide planes, walked in strips of 128 cells (one
+# whole strip and a rest, rows that no workgroup starts with, a plane of one row and a bit)
 GENERAL = [(16, 16, 15), (16, 16, 16), (32, 16, 9), (33, 17, 8), (5, 3, 257)]
 THIN = [(2, 2, 1024), (2, 2, 1025), (5, 1, 1030), (17, 1, 513), (6, 3, 515)]
 FLAT = [(128, 128, 1), (129, 127, 1), (131, 127, 2), (160, 112, 2)]
+WIDE = [(257, 5, 8), (300, 9, 8), (272, 3, 9), (1040, 2, 10)]
 CASES = ([(g, k) for g in GENERAL for k in ("cells_conv", "cells_off")]
          + [(g, k) for g in THIN for k in ("const", "conv", "cells", "tensor")]
-         + [(g, k) for g in FLAT for k in ("const", "conv", "cells", "tensor")])
+         + [(g, k) for g in FLAT for k in ("const", "conv", "cells", "tensor")]
+         + [(g, k) for g in WIDE for k in ("const", "cells")])
 
 
 def operator(pkg, grid, degree, kind, seed=21):
@@ -108,10 +111,11 @@ def test_cg_over_the_choice(pkg, grid, degree, kind):
 
 
 # 1.1 where the general kernel is the right choice or close to it; less where the row kernel (0.87 of
-# the general kernel's time on the plane of more than 4 GiB, 0.80 on the single plane) is
+# the general kernel's time on the plane of more than 4 GiB, 0.80 on the single plane) is, or the
+# matrix-core kernel walking a wide plane in strips (0.67; row after row 1.03)
 TIMES = [((64, 64, 64), 2, "cells_off", 1.1), ((64, 64, 64), 2, "cells_conv", 1.1), ((48, 48, 48), 3, "cells_off", 1.1),
          ((2, 2, 8192), 2, "const", 1.1), ((5, 1, 8192), 3, "cells", 1.1), ((17, 1, 8192), 2, "const", 1.1),
-         ((512, 512, 1), 2, "const", 0.95), ((4096, 2056, 1), 3, "conv", 0.95)]
+         ((512, 512, 1), 2, "const", 0.95), ((4096, 2056, 1), 3, "conv", 0.95), ((2048, 64, 32), 3, "const", 0.85)]
 
 
 @pytest.mark.parametrize("grid,degree,kind,most", TIMES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
