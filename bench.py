@@ -371,8 +371,9 @@ def instationary_leg(pkg, n, k):
     return out
 
 
-# the 64^3 Q3 FP64 apply y = J z (constant kappa): Q3, constant symmetric operator, y = J z
-APPLY_KERNEL = "dg_mfma_kernel<4, 0, 0>"
+# the 64^3 Q3 FP64 apply, as the profiler prints it: Q3, constant symmetric operator, y = J z, no velocity
+# field, four points
+APPLY_KERNEL = "dg_mfma_kernel<4, 0, 0, 0, 4>"
 CALIB_KERNEL = "axpy_kernel<double>"
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "apply_traffic.json")
 
@@ -430,8 +431,22 @@ def profile_summary(d, n, k):
 
 FP64_PEAK = 78.6e12  # MI355X dense FP64 (vector and matrix), FLOP/s
 APPLY_WORKLOADS = {  # grid size (threads) of the apply launches of this benchmark -> workload
-    "131072": "64^3 Q3", "442368": "96^3 Q2", "2097152": "64^3 Q3", "4194304": "64^3 Q3", "995328": "96^3 Q2", "7962624": "96^3 Q2",
-    "56623104": "96^3 Q2"}  # the last: conv_var_kernel, one 64-lane wave per cell
+    # matrix cores: 256 x 4 and 576 x 3 workgroups
+    "262144": "64^3 Q3", "442368": "96^3 Q2",
+    # row kernel (FP32), with and without its walk along z
+    "2097152": "64^3 Q3", "4194304": "64^3 Q3", "995328": "96^3 Q2", "7962624": "96^3 Q2",
+    "56623104": "96^3 Q2"}  # conv_var_kernel, one 64-lane wave per cell
+
+
+def apply_bytes_per_dof(name, k):
+    """Algorithmic bytes per DoF of an apply kernel named as the profiler prints it: z read and y written
+    (and read where y is added to), and the velocity field at its volume and face points."""
+    args = name[name.index("<") + 1:name.rindex(">")].split(", ")
+    if name.startswith("dg_mfma_kernel"):  # <N1, kind, mode, velocity, points>, always FP64
+        mode, vel, m = (int(a) for a in args[2:5])
+        return 16.0 + (8.0 if mode == 1 else 0.0) + (8.0 * (3 * m ** 3 + 6 * m ** 2) / (k + 1) ** 3 if vel else 0.0)
+    es = 8.0 if "double" in args else 4.0
+    return 3 * es + 135 * es / (k + 1) ** 3 if name.startswith("conv_var") else 2 * es
 
 
 def counter_summary(d):
@@ -440,7 +455,7 @@ def counter_summary(d):
     counter sets). Per kernel: median duration, achieved HBM fraction (16 B/DoF FP64, 8 B/DoF
     FP32 over 8 TB/s), VALU busy (SQ_INSTS_VALU x 4 cycles over the 1024 SIMDs' cycles; GRBM_GUI_ACTIVE
     is summed over the 8 XCDs), FP64 utilisation ((2 FMA + ADD + MUL)_F64 x 64 lanes per wave
-    instruction / duration / 78.6 TFLOP/s), LDS busy and bank-conflict cycles (per CU), SALU busy,
+    instruction and 512 per SQ_INSTS_VALU_MFMA_MOPS_F64 / duration / 78.6 TFLOP/s), LDS busy and bank-conflict cycles (per CU), SALU busy,
     instructions per wave, fraction of wave cycles waiting, mean resident waves per CU
     (SQ_WAVE_CYCLES counts quad-cycles: 4 SQ_WAVE_CYCLES / cycles / 256, rocprofv3's own
     OccupancyPercent formula), HBM
@@ -478,16 +493,14 @@ def counter_summary(d):
         wl = APPLY_WORKLOADS[key[1]]
         n, k = (64, 3) if "Q3" in wl else (96, 2)
         N = n ** 3 * (k + 1) ** 3
-        bpd = 16.0 if "double" in s else 8.0
-        if s.startswith("conv_var"):
-            es = 8.0 if "double" in s else 4.0
-            bpd = 3 * es + 135 * es / (k + 1) ** 3
+        bpd = apply_bytes_per_dof(s, k)
         waves = c["SQ_WAVES"]
-        fp64 = 2 * c["SQ_INSTS_VALU_FMA_F64"] + c["SQ_INSTS_VALU_ADD_F64"] + c["SQ_INSTS_VALU_MUL_F64"]
+        fp64 = 64 * (2 * c["SQ_INSTS_VALU_FMA_F64"] + c["SQ_INSTS_VALU_ADD_F64"] + c["SQ_INSTS_VALU_MUL_F64"])
+        fp64 += 512 * c.get("SQ_INSTS_VALU_MFMA_MOPS_F64", 0.0)
         traffic = (2.0 * c["FETCH_SIZE"] + c["WRITE_SIZE"]) * 1024.0 / (bpd * N)
         out.append(
             f"| `{s}` | {wl} | {us:.1f} | {bpd * N / (us * 1e-6) / 8e12:.2f} | "
-            f"{c['SQ_INSTS_VALU'] * 4 / 1024 / cyc:.2f} | {fp64 * 64 / (us * 1e-6) / FP64_PEAK:.2f} | "
+            f"{c['SQ_INSTS_VALU'] * 4 / 1024 / cyc:.2f} | {fp64 / (us * 1e-6) / FP64_PEAK:.2f} | "
             f"{c['SQ_LDS_IDX_ACTIVE'] / 256 / cyc:.2f} | {c['SQ_LDS_BANK_CONFLICT'] / 256 / cyc:.2f} | "
             f"{c['SQ_INSTS_SALU'] / 1024 / cyc:.2f} | {c['SQ_INSTS_VALU'] / waves:.0f} | {c['SQ_INSTS_LDS'] / waves:.0f} | "
             f"{(c['SQ_INSTS_VMEM_RD'] + c['SQ_INSTS_VMEM_WR']) / waves:.0f} | {c['SQ_WAIT_ANY'] / c['SQ_WAVE_CYCLES']:.2f} | "
@@ -496,13 +509,14 @@ def counter_summary(d):
 
 
 def measured_traffic(n, k):
-    """HBM bytes per apply launch from the committed rocprofv3 counter runs (or None)."""
+    """HBM bytes per apply launch from the committed rocprofv3 counter runs, or None where they are of
+    another workload or of another kernel than the one this benchmark runs."""
     try:
         with open(TRAFFIC_FILE) as fh:
             t = json.load(fh)
     except (OSError, ValueError):
         return None
-    return t["traffic_bytes"] if (t.get("n"), t.get("degree")) == (n, k) else None
+    return t["traffic_bytes"] if (t.get("kernel"), t.get("n"), t.get("degree")) == (APPLY_KERNEL, n, k) else None
 
 
 def main():
