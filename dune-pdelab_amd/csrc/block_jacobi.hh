@@ -447,8 +447,10 @@ __global__ __launch_bounds__(256) void bj_dense_setup_kernel(const DGArgs<double
 //            diagonalisation by boundary type only, whose data stay in LDS: W^{-1} r is applied a
 //            second time instead of written and read back, and the dot needs its forward half only
 //            (64^3 Q3, 134 MB per vector: 8 instead of 9 streams, 83 + 101 -> 63 + 95 us, 6.5 and
-//            7.1 TB/s, and the apply that follows finds more of p in the cache, 70 -> 50 us). Vectors
-//            of up to 2^23 elements take BJ_CGR: their p update has the check in it
+//            7.1 TB/s, and the apply that follows finds more of p in the cache, 70 -> 50 us). Q3 only: at
+//            Q1 and Q2 the sweeps, whose waves have idle lanes at Q2, cost more than the stream (96^3 Q2
+//            623 against 612 us per iteration, in FP32 385 against 348; 69^3 Q2 236 against 219; 104^3 Q1
+//            204 against 193). Vectors of up to 2^23 elements take BJ_CGR: their p update has the check in it
 // Every mode returns at once when a state is given and its stop flag state[0] is set (the
 // device-side Krylov loops).
 template <typename T, typename A>

@@ -158,12 +158,14 @@ int launch_n(H* h, const BlockJacobiData& b, const T* data, const BJVec<T, A>& v
   const BJGeom g = geom(h, b.per_cell);
   const long long nb = bj_groups(h, b.fdm);
   if constexpr (MODE == BJ_CGD || MODE == BJ_CGX) {  // bj_cg_recompute() holds
-    if (((long long)g.n[0] * g.n[1]) % BJFdmShape<N1>::CPW == 0)
-      hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, false, true>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0,
-                         h->stream, v, data, g);
-    else
-      hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, false>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0, h->stream,
-                         v, data, g);
+    if constexpr (N1 == 4) {
+      if (((long long)g.n[0] * g.n[1]) % BJFdmShape<N1>::CPW == 0)
+        hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, false, true>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0,
+                           h->stream, v, data, g);
+      else
+        hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, false>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0, h->stream,
+                           v, data, g);
+    }
   } else if (b.fdm && b.per_cell)
     hipLaunchKernelGGL((bj_fdm_kernel<N1, T, A, MODE, true>), dim3(nb), dim3(BJFdmShape<N1>::THREADS), 0, h->stream, v,
                        data, g);
@@ -299,7 +301,7 @@ int bj_launch(H* h, bool trans, int mode, BJVec<T, A> v, int* nparts) {
 
 bool bj_cg_recompute(const H* h, bool trans) {
   const BlockJacobiData& b = h->bj[trans ? 1 : 0];
-  return b.fdm && !b.per_cell;
+  return h->n1 == 4 && b.fdm && !b.per_cell;
 }
 
 template int bj_launch<double, double>(H*, bool, int, BJVec<double, double>, int*);
