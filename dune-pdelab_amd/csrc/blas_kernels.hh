@@ -254,12 +254,15 @@ __global__ __launch_bounds__(kFinalThreads) void cg_pq_kernel(const A* __restric
   }
 }
 
-// Which of an iteration's vectors are left in the 256 MB memory-side cache. x and dinv are read once
-// and stream past it unless all five fit; p, q and z, which the next kernels read again, stay while
-// these three fit; else only p, for the apply. Mixed solve at 64^3 Q3 lognormal (67 MB per vector):
-// z and q streamed, dinv cached 519 ms, z and q kept, dinv streamed 505 ms, dinv cached as well 535 ms.
-// FP64 CG at 64^3 Q3 (134 MB): dinv cached 829 ms, streamed 766 ms; with z and q kept 839 ms. At 72^3 Q2
-// (81 MB) 281, 273 and 290 ms. Mixed solve at 64^3 Q2 (28 MB): all cached 152 ms, as before 157 ms.
+// Which of an iteration's vectors are left in the 256 MB memory-side cache. dinv, read once, streams past
+// it unless all five vectors fit (CG_ALL); q and z, which the next kernels read again, stay with p while
+// these three fit (CG_KEEP); else only p, for the apply (CG_STREAM). x streams in cg_xpupdate_kernel;
+// cg_xpcheck_kernel, for vectors of up to 2^23 elements, leaves all of its own. Each line's times are of one
+// card and one run (the first solve has taken 501 to 537 ms on different cards). Mixed solve at 64^3 Q3
+// lognormal (67 MB per vector): z and q streamed, dinv cached 519 ms, z and q kept, dinv streamed 505 ms,
+// dinv cached as well 535 ms. FP64 CG at 64^3 Q3 (134 MB): dinv cached 829 ms, streamed 766 ms; with z and q
+// kept 839 ms. At 72^3 Q2 (81 MB) 281, 273 and 290 ms. Mixed solve at 64^3 Q2 (28 MB): all cached 152 ms, as
+// before 157 ms.
 enum { CG_STREAM = 0, CG_KEEP = 1, CG_ALL = 2 };
 constexpr int cg_cache(long long bytes) {
   return 5 * bytes <= 224LL << 20 ? CG_ALL : (3 * bytes <= 224LL << 20 ? CG_KEEP : CG_STREAM);

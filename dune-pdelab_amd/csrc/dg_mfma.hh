@@ -24,13 +24,16 @@
 // take the same path. Q2 pads the 4x4 blocks with zeros. mfma_kernel() says which calls come here.
 //
 // Measured (y = J z, three states in turn, row kernel -> this one): 64^3 Q3 76.2 -> 61.6 us (268 MB,
-// 4.4 TB/s; reads 1.17x and writes 1.0x the algorithmic bytes; without memory traffic 31 us, so
-// it is bound by HBM and its latency), lognormal kappa 117 -> 72 us; 96^3 Q2 145 -> 118 us (70 us
-// without memory traffic: 9/16 of the matrix lanes are padding), convection 204 -> 129 us.
+// 4.4 TB/s), lognormal kappa 117 -> 72 us; 96^3 Q2 145 -> 118 us, convection 204 -> 129 us. At 64^3 Q3 it
+// reads 1.33x and writes 1.0x the algorithmic bytes, 1.17x in all, runs at 41 % of the FP64 rate with 10
+// waves per CU, and no unit is busy for more than 40 % of the time: the latency of a step's loads, products
+// and layout changes bounds it. At Q2 9/16 of the matrix lanes are padding.
 // With a velocity field (before: the apply with b = 0, then a kernel of one cell per wave and
 // seven barrier phases over LDS): 64^3 Q2 296 -> 107 us (340 MB, 3.2 TB/s), 40^3 Q3 145 -> 46 us, with
-// cell-wise kappa 141 -> 66 us. Two waves per SIMD hold 170 to 256 registers; three spill and
-// were slower (112 us). Bound by the latency of a step's chain of 93 (Q2) or 120 products.
+// cell-wise kappa 141 -> 66 us. Two waves per SIMD hold 170 to 256 registers (of the Q3 instances six
+// spill 20 to 72 bytes all the same: cell-wise kappa, and diagonal tensors or weightsOff in y +=); three
+// spilled everywhere and were slower (112 us). Bound by the latency of a step's chain of 93 (Q2) or 120
+// products.
 #ifndef PDELAB_DG_MFMA_HH
 #define PDELAB_DG_MFMA_HH
 
@@ -102,9 +105,9 @@ struct MfmaArgs {
 enum { MFMA_CONST = 0, MFMA_WEIGHT = 1, MFMA_GENERAL = 2, MFMA_CONV = 3, MFMA_TENSOR = 4 };
 constexpr int mfma_row(bool tensor) { return tensor ? 6 : 4; }  // values of a cell's row
 
-// Waves per SIMD the register allocation aims at: no instance spills. (With 96 bytes of scratch
-// the face-weight Q3 kernel took 97 instead of 76 us at 64^3, and 72 bytes cost the fused-dot
-// Q2 one 5 of 17 us at 32^3.)
+// Waves per SIMD the register allocation aims at without a velocity field: no vector register goes to
+// scratch. (With 96 bytes of it the face-weight Q3 kernel took 97 instead of 76 us at 64^3, and 72 bytes
+// cost the fused-dot Q2 one 5 of 17 us at 32^3. Up to 130 scalar registers are parked in vector lanes.)
 template <int N1, int KIND, int MODE>
 constexpr int mfma_waves() {
   if (KIND == MFMA_GENERAL) return 2;

@@ -740,11 +740,12 @@ static int cg_loop(H* h, T* x, T* b, T* p, T* q, T* z, const Prec<T>& P, bool tr
 // Workspace slots base, base+1 (p, q).
 //
 // The loop runs on the device: per iteration the apply (with the fused p.q partials),
-// the update of r (with the r.r and z.r partials), the Iteration::step check and the
-// update of x and the direction are enqueued without waiting; the check kernel raises a
-// device flag at the iteration where dune-istl's stopping rule fires and every later
-// kernel of the loop returns immediately, so the state is exactly the one at that
-// iteration. The host reads the flag back every kCheckEvery iterations.
+// the update of r (with the r.r and z.r partials; with point Jacobi it holds z = dinv r until
+// the loop ends), the Iteration::step check and the update of x and the direction are enqueued
+// without waiting. The check, a launch of its own or part of the x/p update, raises a device flag
+// at the iteration where dune-istl's stopping rule fires and every later kernel of the loop returns
+// immediately, so the state is exactly the one at that iteration. Every kCheckEvery iterations the
+// host reads the flag of kCheckEvery iterations earlier.
 template <typename T, typename A>
 static int cg_solve(H* h, T* x, T* b, double reduction, int maxit, int precond, bool trans, int base,
                     pdelab_linear_solver_result* res) {
